@@ -39,7 +39,7 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
 }
 
 template <bool TA, bool TB, int BM, int BN, bool SPLIT = false>
-__device__ __forceinline__ void gemm_body(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles,
+__device__ __forceinline__ void gemm_lds_body(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles,
                                           const Bases& bases, int split = 1, double* __restrict__ ws = nullptr) {
   constexpr int BK = 16;
   // LDS layout follows each operand's memory order so that both the global
@@ -180,19 +180,202 @@ __device__ __forceinline__ void gemm_body(const GemmProb* __restrict__ probs, co
       }
 }
 
-// 64x64 tiles: four blocks per CU (LDS 38 KB, ~120 registers).
-template <bool TA, bool TB>
+
+// The same product without LDS.  An FP64 MFMA keeps its SIMD busy for 64
+// cycles and consumes two 512-byte fragments, so the matrix cores are fed
+// from L1/L2 directly and no wave ever waits at a barrier.  Each lane loads
+// its own fragment elements: lane (lr, lk) = (lane % 16, lane / 16) holds, for
+// the sub-steps s = 0..3 of a 16-deep slab, k = 4 lk + s of row lr of each
+// 16-row fragment.  The order of k inside a slab is free as long as both
+// operands use it, and this one lets an operand whose k is contiguous (op(A) =
+// A^T, op(B) = B) be read 16 bytes at a time (VEC: its offset and leading
+// dimension are even); an operand with contiguous rows reads 128-byte segments.
+// A half of the slab (two sub-steps) is reloaded for the next slab as soon as
+// its MFMAs are issued, two to four thousand cycles before its use.  Rows past
+// the edge are clamped (their results are not stored); the last, partial
+// slab loads zeros past K.
+// Alone on the chip (TFLOP/s; LDS kernels before -> this one, 78.6 peak):
+// 4096^3 NT 58 -> 65, NN 58 -> 67, TN 51 -> 64; 4096 x 1920 x 4096 NT 53 -> 59,
+// NN 54 -> 60, TN 47 -> 66; 64x64 tiles NT 46 -> 56.  With 64x64 tiles and k
+// contiguous in both operands the 16-line loads bound it (38 against 52
+// TFLOP/s), so that form keeps the LDS kernel above.
+template <bool KC, bool VEC, int T>
+__device__ __forceinline__ void load_half(double (&f)[T][4], const uint32_t (&off)[T], const char* base, int64_t ldb,
+                                          int h) {
+  if constexpr (KC) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if constexpr (VEC) {
+        const double2 x = *(const double2*)(base + off[t] + h * 16);
+        f[t][2 * h] = x.x;
+        f[t][2 * h + 1] = x.y;
+      } else {
+        f[t][2 * h] = *(const double*)(base + off[t] + h * 16);
+        f[t][2 * h + 1] = *(const double*)(base + off[t] + h * 16 + 8);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const char* b = base + (2 * h + u) * ldb;
+#pragma unroll
+      for (int t = 0; t < T; ++t) f[t][2 * h + u] = *(const double*)(b + off[t]);
+    }
+  }
+}
+// The partial slab: k = 4 lk + s < rem.
+template <bool KC, int T>
+__device__ __forceinline__ void load_tail(double (&f)[T][4], const uint32_t (&off)[T], const char* base, int64_t ldb,
+                                          int lk, int rem) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const bool in = 4 * lk + s < rem;
+#pragma unroll
+    for (int t = 0; t < T; ++t) f[t][s] = in ? *(const double*)(base + off[t] + (KC ? (int64_t)s * 8 : s * ldb)) : 0.0;
+  }
+}
+
+template <bool TA, bool TB, bool VEC, int TM, int TN, bool SPLIT = false>
+__device__ __forceinline__ void gemm_reg_body(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles,
+                                              const Bases& bases, int split = 1, double* __restrict__ ws = nullptr) {
+  constexpr int BM = 32 * TM, BN = 32 * TN;  // four waves, 2 x 2
+  constexpr bool AKC = TA, BKC = !TB;        // k contiguous
+  const GemmTile t = tiles[SPLIT ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x)];
+  const GemmProb P = probs[t.prob];
+  const int M = P.M, N = P.N;
+  const int m0 = t.tm * BM, n0 = t.tn * BN;
+  int kb = 0, K = P.K;  // this block's K range [kb, K): the zeros of a triangular operand are skipped
+  if (P.kmode == 1)
+    kb = min(K, n0);
+  else if (P.kmode == 2)
+    kb = min(K, m0);
+  else if (P.kmode == 3)
+    K = min(K, m0 + BM);
+  if constexpr (SPLIT) {
+    const int kc = ((K - kb + split - 1) / split + 15) / 16 * 16;
+    const int k0 = min(K, kb + t.pad * kc);
+    K = min(K, k0 + kc);
+    kb = k0;
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lr = lane & 15, lk = lane >> 4;
+  const int wm = (wave & 1) * 16 * TM, wn = (wave >> 1) * 16 * TN;
+  // wave-uniform bases at the tile's first row and column and at kb; the lane
+  // offsets stay below 2^32 (128 rows or 12 columns of one front)
+  const int64_t lda = (int64_t)P.lda * 8, ldb = (int64_t)P.ldb * 8;
+  const char* pa = (const char*)(bases.p[P.a_base] + P.a_off) + (AKC ? m0 * lda + kb * 8ll : m0 * 8ll + kb * lda);
+  const char* pb = (const char*)(bases.p[P.b_base] + P.b_off) + (BKC ? n0 * ldb + kb * 8ll : n0 * 8ll + kb * ldb);
+  uint32_t oa[TM], ob[TN];
+#pragma unroll
+  for (int y = 0; y < TM; ++y) {
+    const int r = min(wm + y * 16 + lr, M - 1 - m0);
+    oa[y] = AKC ? (uint32_t)(r * (uint32_t)lda + lk * 32) : (uint32_t)(r * 8 + lk * 4 * (uint32_t)lda);
+  }
+#pragma unroll
+  for (int x = 0; x < TN; ++x) {
+    const int c = min(wn + x * 16 + lr, N - 1 - n0);
+    ob[x] = BKC ? (uint32_t)(c * (uint32_t)ldb + lk * 32) : (uint32_t)(c * 8 + lk * 4 * (uint32_t)ldb);
+  }
+  const int64_t sa = AKC ? 128 : 16 * lda, sb = BKC ? 128 : 16 * ldb;
+  d4 acc[TN][TM];
+#pragma unroll
+  for (int x = 0; x < TN; ++x)
+#pragma unroll
+    for (int y = 0; y < TM; ++y) acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+  double fa[TM][4], fb[TN][4];
+  auto mul = [&](int h) {
+#pragma unroll
+    for (int s = 2 * h; s < 2 * h + 2; ++s)
+#pragma unroll
+      for (int x = 0; x < TN; ++x)
+#pragma unroll
+        for (int y = 0; y < TM; ++y)
+          acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[x][s], fa[y][s], acc[x][y], 0, 0, 0);
+  };
+  const int nk = max(K - kb, 0) >> 4, rem = max(K - kb, 0) & 15;
+  if (nk > 0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      load_half<AKC, VEC, TM>(fa, oa, pa, lda, h);
+      load_half<BKC, VEC, TN>(fb, ob, pb, ldb, h);
+    }
+    for (int kt = 1; kt < nk; ++kt) {
+      pa += sa;
+      pb += sb;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        mul(h);
+        __builtin_amdgcn_sched_barrier(0);
+        load_half<AKC, VEC, TM>(fa, oa, pa, lda, h);
+        load_half<BKC, VEC, TN>(fb, ob, pb, ldb, h);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    mul(0);
+    mul(1);
+    pa += sa;
+    pb += sb;
+  }
+  if (rem) {
+    load_tail<AKC, TM>(fa, oa, pa, lda, lk, rem);
+    load_tail<BKC, TN>(fb, ob, pb, ldb, lk, rem);
+    mul(0);
+    mul(1);
+  }
+  if constexpr (SPLIT) {
+    double* w = ws + (int64_t)blockIdx.x * (BM * BN);
+#pragma unroll
+    for (int x = 0; x < TN; ++x)
+#pragma unroll
+      for (int y = 0; y < TM; ++y)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) w[(wm + y * 16 + lr) + (wn + x * 16 + lk + 4 * v) * BM] = acc[x][y][v];
+    return;
+  }
+  // A and C may be the same memory (the in-place panel solve, one tile
+  // column): every wave has read its rows of A before any wave writes them
+  __syncthreads();
+  double* C = bases.p[P.c_base] + P.c_off;
+  const double alpha = P.alpha, beta = P.beta;
+  const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
+  // lower problems: the part of a tile above the diagonal is left
+  // untouched (it is never read, and stays as initialised)
+  const bool straddles = P.lower && m0 < n0 + BN;
+#pragma unroll
+  for (int x = 0; x < TN; ++x)
+#pragma unroll
+    for (int y = 0; y < TM; ++y)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int m = m0 + wm + y * 16 + lr;
+        const int n = n0 + wn + x * 16 + lk + 4 * v;
+        if ((interior || (m < M && n < N)) && !(straddles && m < n)) {
+          double* c = C + m + (int64_t)n * P.ldc;
+          const double r = alpha * acc[x][y][v];
+          *c = (beta == 0.0) ? r : r + beta * (*c);
+        }
+      }
+}
+
+// 64x64 tiles.
+template <bool TA, bool TB, bool VEC>
 __global__ __launch_bounds__(256) void gemm64_kernel(const GemmProb* __restrict__ probs,
                                                      const GemmTile* __restrict__ tiles, Bases bases) {
-  gemm_body<TA, TB, 64, 64>(probs, tiles, bases);
+  if constexpr (TA && !TB)
+    gemm_lds_body<TA, TB, 64, 64>(probs, tiles, bases);
+  else
+    gemm_reg_body<TA, TB, VEC, 2, 2>(probs, tiles, bases);
 }
 
 // Split-K partial tiles (64x64) and their ordered sum.
-template <bool TA, bool TB>
+template <bool TA, bool TB, bool VEC>
 __global__ __launch_bounds__(256) void gemm64_split_kernel(const GemmProb* __restrict__ probs,
                                                            const GemmTile* __restrict__ tiles, Bases bases, int split,
                                                            double* __restrict__ ws) {
-  gemm_body<TA, TB, 64, 64, true>(probs, tiles, bases, split, ws);
+  if constexpr (TA && !TB)
+    gemm_lds_body<TA, TB, 64, 64, true>(probs, tiles, bases, split, ws);
+  else
+    gemm_reg_body<TA, TB, VEC, 2, 2, true>(probs, tiles, bases, split, ws);
 }
 
 // Block b: C tile of tiles[b * split] = alpha * sum_q partial[b * split + q]
@@ -218,13 +401,15 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmProb* __res
   }
 }
 
-// 128x128 tiles (each wave 64x64: half the LDS reads per MFMA): two blocks
-// per CU (LDS 74 KB); the register budget is pinned to two waves per SIMD,
-// without it the compiler takes ~360 registers and one wave.
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm128_kernel(
-    const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles, Bases bases) {
-  gemm_body<TA, TB, 128, 128>(probs, tiles, bases);
+// Large tiles: 128x64 at three waves per SIMD (64x128 where op(A) = A^T and
+// op(B) = B^T: the operand with contiguous k takes the short edge, 67 against 59
+// TFLOP/s at 4096^3), and 128x128 at two waves where k is contiguous in both
+// operands (their 16-line loads want the larger tile: 64 against 50; elsewhere
+// 128x64 leads 128x128, 65 against 61 NT and 67 against 63 NN).
+template <bool TA, bool TB, bool VEC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TA && !TB ? 2 : 3, TA && !TB ? 2 : 3))) void
+gemm128_kernel(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles, Bases bases) {
+  gemm_reg_body<TA, TB, VEC, (TA && TB) ? 2 : 4, TA ? 4 : 2>(probs, tiles, bases);
 }
 
 // y = alpha op(A) x + beta y for N <= kGemvMaxN columns (solves with few
@@ -322,39 +507,37 @@ void launch_gemm(const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned ld
       hipLaunchKernelGGL(gemv_kernel<false>, grid, block, 0, s, g.d_probs, g.d_tiles, b);
     return;
   }
+  // VEC matters only where k is contiguous in an operand
+#define SPDE_GEMM_FORM(K, ...)                                        \
+  do {                                                                \
+    const bool vec = g.vec;                                           \
+    if (!g.ta && g.tb)                                                \
+      hipLaunchKernelGGL((K<false, true, true>), __VA_ARGS__);        \
+    else if (!g.ta && vec)                                            \
+      hipLaunchKernelGGL((K<false, false, true>), __VA_ARGS__);       \
+    else if (!g.ta)                                                   \
+      hipLaunchKernelGGL((K<false, false, false>), __VA_ARGS__);      \
+    else if (!g.tb && vec)                                            \
+      hipLaunchKernelGGL((K<true, false, true>), __VA_ARGS__);        \
+    else if (!g.tb)                                                   \
+      hipLaunchKernelGGL((K<true, false, false>), __VA_ARGS__);       \
+    else if (vec)                                                     \
+      hipLaunchKernelGGL((K<true, true, true>), __VA_ARGS__);         \
+    else                                                              \
+      hipLaunchKernelGGL((K<true, true, false>), __VA_ARGS__);        \
+  } while (0)
   if (g.split > 1) {
     double* ws = b.ws + g.ws_off;
-    if (!g.ta && !g.tb)
-      hipLaunchKernelGGL((gemm64_split_kernel<false, false>), grid, block, 0, s, g.d_probs, g.d_tiles, b, g.split, ws);
-    else if (!g.ta && g.tb)
-      hipLaunchKernelGGL((gemm64_split_kernel<false, true>), grid, block, 0, s, g.d_probs, g.d_tiles, b, g.split, ws);
-    else if (g.ta && !g.tb)
-      hipLaunchKernelGGL((gemm64_split_kernel<true, false>), grid, block, 0, s, g.d_probs, g.d_tiles, b, g.split, ws);
-    else
-      hipLaunchKernelGGL((gemm64_split_kernel<true, true>), grid, block, 0, s, g.d_probs, g.d_tiles, b, g.split, ws);
+    SPDE_GEMM_FORM(gemm64_split_kernel, grid, block, 0, s, g.d_probs, g.d_tiles, b, g.split, ws);
     hipLaunchKernelGGL(split_reduce_kernel, dim3(g.ntiles / g.split), block, 0, s, g.d_probs, g.d_tiles, b, g.split,
                        ws);
     return;
   }
-  if (g.tile == 128) {
-    if (!g.ta && !g.tb)
-      hipLaunchKernelGGL((gemm128_kernel<false, false>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-    else if (!g.ta && g.tb)
-      hipLaunchKernelGGL((gemm128_kernel<false, true>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-    else if (g.ta && !g.tb)
-      hipLaunchKernelGGL((gemm128_kernel<true, false>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-    else
-      hipLaunchKernelGGL((gemm128_kernel<true, true>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-  } else {
-    if (!g.ta && !g.tb)
-      hipLaunchKernelGGL((gemm64_kernel<false, false>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-    else if (!g.ta && g.tb)
-      hipLaunchKernelGGL((gemm64_kernel<false, true>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-    else if (g.ta && !g.tb)
-      hipLaunchKernelGGL((gemm64_kernel<true, false>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-    else
-      hipLaunchKernelGGL((gemm64_kernel<true, true>), grid, block, lds, s, g.d_probs, g.d_tiles, b);
-  }
+  if (g.tile == 128)
+    SPDE_GEMM_FORM(gemm128_kernel, grid, block, lds, s, g.d_probs, g.d_tiles, b);
+  else
+    SPDE_GEMM_FORM(gemm64_kernel, grid, block, lds, s, g.d_probs, g.d_tiles, b);
+#undef SPDE_GEMM_FORM
 }
 
 // ------------------------------------------------ diagonal block Cholesky
@@ -647,12 +830,13 @@ extern "C" int spde_debug_gemm(int ta, int tb, int M, int N, int K, double alpha
   P.alpha = alpha;
   P.beta = beta;
   std::vector<GemmTile> tiles;
-  for (int a = 0; a < (M + tile - 1) / tile; ++a)
-    for (int b = 0; b < (N + tile - 1) / tile; ++b) tiles.push_back({0, a, b, 0});
   GemmLaunch g;
   g.tile = tile;
   g.ta = ta != 0;
   g.tb = tb != 0;
+  g.vec = !((uintptr_t)A & 15) && !((uintptr_t)B & 15) && !(lda & 1) && !(ldb & 1);
+  for (int a = 0; a < (M + g.tile_m() - 1) / g.tile_m(); ++a)
+    for (int b = 0; b < (N + g.tile_n() - 1) / g.tile_n(); ++b) tiles.push_back({0, a, b, 0});
   g.ntiles = (int)tiles.size();
   SPDE_HIP(hipMalloc((void**)&g.d_probs, sizeof(GemmProb)));
   SPDE_HIP(hipMalloc((void**)&g.d_tiles, sizeof(GemmTile) * tiles.size()));

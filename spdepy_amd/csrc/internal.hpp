@@ -51,7 +51,10 @@ struct GemmTile {
 // A batched GEMM launch: problems + tile list (device), transposition flags.
 struct GemmLaunch {
   bool ta = false, tb = false;
-  int tile = 64;                 // block tile edge (64 or 128), chosen when finalised
+  int tile = 64;                 // longer edge of a block tile (64 or 128), chosen when finalised
+  int tile_m() const { return tile == 128 && ta && tb ? 64 : tile; }  // rows and columns of a tile
+  int tile_n() const { return tile == 128 && !ta ? 64 : tile; }
+  bool vec = false;              // operands with contiguous k: even offsets and leading dimensions (16-byte loads)
   int ntiles = 0, nprobs = 0;
   GemmProb* d_probs = nullptr;
   GemmTile* d_tiles = nullptr;
@@ -135,9 +138,22 @@ struct Slot {
 };
 
 struct NodeDev {            // per-node table on the device
-  int64_t foff, zoff, voff, relpos_off;
-  int32_t start, p, n, parent, nb, level, pad0, pad1;
+  int64_t foff, zoff, voff, relpos_off;  // foff, zoff: device layout
+  int32_t start, p, n, parent, nb, level, ld, pp;
 };
+
+// Device layout of one front and its Z: the own columns are padded to pp (a
+// multiple of kFrontPad), the boundary rows and columns follow at pp, and the
+// leading dimension is a multiple of 16 doubles, so that every block of a
+// front starts on a 128-byte line: fragment loads touch whole lines, operands
+// with contiguous k are read 16 bytes at a time, and no two 64-row tiles
+// share a line.  The symbolic analysis and the exported plan keep the compact
+// n x n fronts.  (The pad rows and columns hold zeros or values nothing reads.)
+struct FrontLay {
+  int64_t foff, zoff;
+  int32_t ld, pp;
+};
+constexpr int kFrontPad = 64;
 
 }  // namespace spde
 
@@ -146,7 +162,7 @@ struct spde_plan {
   spde::Structure st;
   spde::Symbolic sym;
   std::vector<int64_t> map;      // scatter map (front offsets, -1 upper)
-  std::vector<int64_t> mapsym;   // map of the lower mirror for every entry
+
   bool host_only = true;
   int nslots = 0;
   // device structure
@@ -176,6 +192,8 @@ struct spde_plan {
   int32_t* d_sprow = nullptr;     // one-slice plans: row and column of each entry (Kronecker kernels)
   int32_t* d_spcol = nullptr;
   int64_t work_doubles = 0;       // per-slot workspace size
+  std::vector<spde::FrontLay> lay;  // device layout per node
+  int64_t lay_front = 0, lay_z = 0;  // arena sizes (doubles) of that layout
   std::vector<spde::Slot> slots;
   std::vector<spde::LevelPlan> levels;
   std::vector<spde::GemmLaunch> trtri;  // per recursion height: pairs (X, Z2)

@@ -62,10 +62,10 @@ __global__ __launch_bounds__(256) void zero_lower_kernel(const NodeDev* __restri
   const NodeDev nd = nodes[t.x];
   double* f = F + nd.foff;
   const int i = t.y * 64 + (threadIdx.x & 63);
-  if (i >= nd.n) return;
+  if (i >= nd.pp + nd.nb) return;
   for (int jj = threadIdx.x >> 6; jj < 64; jj += 4) {
     const int j = t.z * 64 + jj;
-    if (j <= i) f[i + (int64_t)j * nd.n] = 0.0;
+    if (j <= i) f[i + (int64_t)j * nd.ld] = 0.0;
   }
 }
 
@@ -153,7 +153,10 @@ __global__ __launch_bounds__(256) void fwd_gather_kernel(const int32_t* __restri
     const NodeDev cd = nodes[ch];
     const int32_t* rp = relpos + cd.relpos_off;
     const double* u = vec + cd.voff * nrhs + (int64_t)c * cd.n;
-    for (int r = threadIdx.x; r < cd.nb; r += 256) v[rp[r]] += u[cd.p + r];
+    for (int r = threadIdx.x; r < cd.nb; r += 256) {
+      const int q = rp[r];  // position in the padded front; v has no padding
+      v[q < nd.pp ? q : q - nd.pp + nd.p] += u[cd.p + r];
+    }
     __syncthreads();
   }
 }
@@ -197,7 +200,7 @@ __global__ __launch_bounds__(256) void sigma_gather_kernel(const int32_t* __rest
   const int i0 = tt.y * 64, j0 = tt.z * 64;
   const bool diag = tt.y == tt.z;
   const double* src = S + pa.foff;
-  const int64_t pn = pa.n;
+  const int64_t pn = pa.ld;
   const int tid = threadIdx.x, u = tid & 63, w0 = tid >> 6;
   // parent positions of the tile's rows and columns (-1 outside the block)
   if (tid < 64) rpi[tid] = (i0 + tid < b) ? rp[i0 + tid] : -1;
@@ -210,12 +213,12 @@ __global__ __launch_bounds__(256) void sigma_gather_kernel(const int32_t* __rest
     const int jj = w0 + 4 * t, pj = rpj[jj];
     v[t] = (pi >= 0 && pj >= 0 && (!diag || u >= jj)) ? src[pi + (int64_t)pj * pn] : 0.0;
   }
-  double* dst = S + nd.foff + nd.p + (int64_t)nd.p * nd.n;
+  double* dst = S + nd.foff + nd.pp + (int64_t)nd.pp * nd.ld;
   const int i = i0 + u;
 #pragma unroll
   for (int t = 0; t < 16; ++t) {
     const int jj = w0 + 4 * t, j = j0 + jj;
-    if (i < b && j < b && (!diag || u >= jj)) dst[i + (int64_t)j * nd.n] = v[t];
+    if (i < b && j < b && (!diag || u >= jj)) dst[i + (int64_t)j * nd.ld] = v[t];
     tile[u][jj] = v[t];
   }
   __syncthreads();
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(256) void sigma_gather_kernel(const int32_t* __rest
 #pragma unroll
   for (int t = 0; t < 16; ++t) {
     const int c = w0 + 4 * t, col = i0 + c;
-    if (row < b && col < b && (!diag || u < c)) dst[row + (int64_t)col * nd.n] = tile[c][u];
+    if (row < b && col < b && (!diag || u < c)) dst[row + (int64_t)col * nd.ld] = tile[c][u];
   }
 }
 

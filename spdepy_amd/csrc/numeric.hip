@@ -46,6 +46,43 @@ __global__ void clear_status_kernel(int* status) {
   if (threadIdx.x == 0) status[threadIdx.x] = 0;
 }
 
+// Device layout of the fronts and Z blocks (FrontLay).
+void build_layout(spde_plan* pl) {
+  const Symbolic& sym = pl->sym;
+  pl->lay.resize(sym.nodes.size());
+  int64_t foff = 0, zoff = 0;
+  for (size_t q = 0; q < sym.nodes.size(); ++q) {
+    const Node& nd = sym.nodes[q];
+    FrontLay& f = pl->lay[q];
+    f.pp = (nd.p + kFrontPad - 1) / kFrontPad * kFrontPad;
+    const int nf = f.pp + (int)nd.B.size();
+    f.ld = (nf + 15) / 16 * 16;
+    f.foff = foff;
+    f.zoff = zoff;
+    foff += (int64_t)f.ld * nf;
+    zoff += (int64_t)f.pp * f.pp;
+  }
+  pl->lay_front = foff;
+  pl->lay_z = zoff;
+}
+
+// Scatter map of the device layout from the compact one.
+std::vector<int64_t> layout_map(const spde_plan* pl) {
+  const Symbolic& sym = pl->sym;
+  const Structure& st = pl->st;
+  std::vector<int64_t> map(pl->map.size(), -1);
+  for (size_t r = 0; r + 1 < st.indptr.size(); ++r)
+    for (int64_t e = st.indptr[r]; e < st.indptr[r + 1]; ++e) {
+      if (pl->map[e] < 0) continue;
+      const int q = sym.col_node[sym.iperm[st.indices[e]]];
+      const Node& nd = sym.nodes[q];
+      const FrontLay& f = pl->lay[q];
+      const int64_t at = pl->map[e] - nd.foff, row = at % nd.n(), col = at / nd.n();
+      map[e] = f.foff + (row < nd.p ? row : row - nd.p + f.pp) + col * f.ld;
+    }
+  return map;
+}
+
 // Device-side per-level index tables that are not part of LevelPlan.
 struct LevelDev {
   int32_t* d_nodes = nullptr;
@@ -119,9 +156,9 @@ int validate(const GemmLaunch& g, const ArenaSizes& a, const char* what) {
 
 ArenaSizes arena_sizes(const spde_plan* pl, int nrhs) {
   ArenaSizes a;
-  a.sz[kFront] = pl->sym.front_doubles;
-  a.sz[kZ] = pl->sym.z_doubles;
-  a.sz[kSigma] = pl->sym.front_doubles;
+  a.sz[kFront] = pl->lay_front;
+  a.sz[kZ] = pl->lay_z;
+  a.sz[kSigma] = pl->lay_front;
   a.sz[kWork] = pl->work_doubles;
   a.sz[kVec] = pl->sym.vec_doubles * nrhs;
   a.sz[kX] = pl->sym.n * nrhs;
@@ -179,11 +216,10 @@ void add_prob(GemmLaunch& g, const GemmProb& P, bool lower, double flop_scale = 
   g.bytes += 8.0 * (P.M * (double)P.K + P.N * (double)P.K + cmn * (P.beta != 0.0 ? 2.0 : 1.0));
 }
 
-// Tile edge of a launch: 128 when the launch has no lower-triangular
-// problem, a mean depth K of at least 256 and >= 512 tiles of 128 (two
-// rounds of the chip at two blocks per CU); else 64 (short or triangular
-// problems keep more blocks in flight and waste less on the diagonal).
-// Then the tile list (tiles strictly above the diagonal of a lower problem
+// A launch takes the large tiles when the mean depth K is at least 128 and
+// they fill the chip's block slots once (768 of 128x64, three per CU;
+// 512 of 128x128, two per CU); else 64 (more blocks in flight, less waste at
+// the edges).  Then the tile list (tiles strictly above the diagonal of a lower problem
 // are skipped).
 void make_tiles(GemmLaunch& g, int force_tile) {
   // few right-hand sides: row blocks of 64 (A not transposed) or groups of 4
@@ -202,37 +238,38 @@ void make_tiles(GemmLaunch& g, int force_tile) {
       for (int a = 0; a < (g.h_probs[i].M + rows - 1) / rows; ++a) g.h_tiles.push_back({(int32_t)i, a, 0, 0});
     return;
   }
-  int64_t t128 = 0;
-  double ksum = 0.0;
-  bool any_lower = false;
-  int64_t t128_lower = 0;  // tiles of 128 actually launched (on or below the diagonal of lower problems)
+  // 16-byte loads of operands with contiguous k (op(A) = A^T, op(B) = B)
+  g.vec = true;
   for (const GemmProb& P : g.h_probs) {
-    const int64_t tm = (P.M + 127) / 128, tn = (P.N + 127) / 128;
-    t128 += tm * tn;
-    t128_lower += P.lower ? (tm <= tn ? tm * (tm + 1) / 2 : tm * tn - tn * (tn - 1) / 2) : tm * tn;
-    ksum += P.K;
-    any_lower = any_lower || P.lower;
+    if (g.ta) g.vec = g.vec && !(P.a_off & 1) && !(P.lda & 1);
+    if (!g.tb) g.vec = g.vec && !(P.b_off & 1) && !(P.ldb & 1);
   }
-  // lower problems: 128 only when the launch still has two full rounds of
-  // 128-tiles (the diagonal tiles do redundant work above the diagonal)
-  const bool deep = !g.h_probs.empty() && ksum / g.h_probs.size() >= 256.0;
-  const bool big = deep && (any_lower ? t128_lower >= 1024 : t128 >= 512);
-  g.tile = force_tile ? force_tile : (big ? 128 : 64);
+  g.tile = 128;
+  const int64_t BM = g.tile_m(), BN = g.tile_n();
+  int64_t big = 0;  // large tiles that would be launched (on or below the diagonal of lower problems)
+  double ksum = 0.0;
+  for (const GemmProb& P : g.h_probs) {
+    const int64_t tm = (P.M + BM - 1) / BM, tn = (P.N + BN - 1) / BN;
+    for (int64_t a = 0; a < tm; ++a) big += P.lower ? std::min(tn, ((a + 1) * BM + BN - 1) / BN) : tn;
+    ksum += P.K;
+  }
+  const bool deep = !g.h_probs.empty() && ksum / g.h_probs.size() >= 128.0;
+  g.tile = force_tile ? force_tile : (deep && big >= (BM * BN == 128 * 64 ? 768 : 512) ? 128 : 64);
   g.h_tiles.clear();
-  const int T = g.tile;
+  const int T = g.tile_m(), TN = g.tile_n();
   for (size_t i = 0; i < g.h_probs.size(); ++i) {
     const GemmProb& P = g.h_probs[i];
-    const int tm = (P.M + T - 1) / T, tn = (P.N + T - 1) / T;
+    const int tm = (P.M + T - 1) / T, tn = (P.N + TN - 1) / TN;
     for (int a = 0; a < tm; ++a)
       for (int b = 0; b < tn; ++b)
-        if (!P.lower || a >= b) g.h_tiles.push_back({(int32_t)i, a, b, 0});
+        if (!P.lower || (a + 1) * T > b * TN) g.h_tiles.push_back({(int32_t)i, a, b, 0});
   }
   // deepest tiles first: the blocks dispatched last are the shortest, which
   // shortens the launch's final, partly filled round
   auto depth = [&](const GemmTile& t) {
     const GemmProb& P = g.h_probs[t.prob];
     int kb = 0, ke = P.K;
-    if (P.kmode == 1) kb = std::min(P.K, t.tn * T);
+    if (P.kmode == 1) kb = std::min(P.K, t.tn * TN);
     if (P.kmode == 2) kb = std::min(P.K, t.tm * T);
     if (P.kmode == 3) ke = std::min(P.K, (t.tm + 1) * T);
     return ke - kb;
@@ -286,7 +323,8 @@ int build_factor_plan(spde_plan* pl) {
         const int di = (int)L.h_ext[s].size();
         int split = 0;  // relpos increases: the first `split` columns map into the parent's own columns
         while (split < b && c.relpos[split] < nd.p) ++split;
-        L.h_ext[s].push_back({c.foff, nd.foff, c.relpos_off, c.n(), c.p, nd.n(), b, split, 0});
+        const FrontLay &cl = pl->lay[nd.child[s]], &fl = pl->lay[id];
+        L.h_ext[s].push_back({cl.foff, fl.foff, c.relpos_off, cl.ld, cl.pp, fl.ld, b, split, 0});
         const int nt = (b + 63) / 64;
         for (int a = 0; a < nt; ++a)
           for (int bb = 0; bb <= a; ++bb) {
@@ -322,13 +360,16 @@ int build_factor_plan(spde_plan* pl) {
         for (int id : L.nodes) {
           const Node& nd = sym.nodes[id];
           if (nd.p <= k0) continue;
-          const int n = nd.n(), kb = std::min(NB, nd.p - k0);
-          pd.push_back({nd.foff, nd.zoff, n, nd.p, k0, kb, id, nd.start + k0});
-          const int M = n - k0 - kb;
-          const int64_t off = nd.foff + (k0 + kb) + (int64_t)k0 * n;
+          const FrontLay& f = pl->lay[id];
+          const int n = f.ld, kb = std::min(NB, nd.p - k0);
+          pd.push_back({f.foff, f.zoff, n, f.pp, k0, kb, id, nd.start + k0});
+          // rows below the block: the own rows, then (past the padding) the boundary
+          const int r0 = k0 + kb < nd.p ? k0 + kb : f.pp;
+          const int M = f.pp + (int)nd.B.size() - r0;
+          const int64_t off = f.foff + r0 + (int64_t)k0 * n;
           // in place (kb <= 64: one tile column); W is lower triangular
           add_prob(st.panel,
-                   prob(kFront, off, n, kZ, nd.zoff + k0 + (int64_t)k0 * nd.p, nd.p, kFront, off, n, M, kb, kb, 1.0, 0.0),
+                   prob(kFront, off, n, kZ, f.zoff + k0 + (int64_t)k0 * f.pp, f.pp, kFront, off, n, M, kb, kb, 1.0, 0.0),
                    false, 0.5);
         }
         st.npotrf = (int)pd.size();
@@ -352,9 +393,10 @@ int build_factor_plan(spde_plan* pl) {
       for (int id : L.nodes) {
         const Node& nd = sym.nodes[id];
         if (nd.p <= m) continue;
-        const int n = nd.n(), M = n - m, N = std::min(b, nd.p) - m, K = m - a;
-        const int64_t ab = nd.foff + m + (int64_t)a * n;
-        add_prob(st.update, prob(kFront, ab, n, kFront, ab, n, kFront, nd.foff + m + (int64_t)m * n, n, M, N, K, -1.0, 1.0),
+        const FrontLay& f = pl->lay[id];
+        const int n = f.ld, M = f.pp + (int)nd.B.size() - m, N = std::min(b, nd.p) - m, K = m - a;
+        const int64_t ab = f.foff + m + (int64_t)a * n;
+        add_prob(st.update, prob(kFront, ab, n, kFront, ab, n, kFront, f.foff + m + (int64_t)m * n, n, M, N, K, -1.0, 1.0),
                  true);
       }
       rc = finalize(st.update, &pl->split_fs);
@@ -370,11 +412,12 @@ int build_factor_plan(spde_plan* pl) {
     L.syrk.tb = true;
     for (int id : L.nodes) {
       const Node& nd = sym.nodes[id];
-      const int n = nd.n(), b = (int)nd.B.size();
+      const FrontLay& f = pl->lay[id];
+      const int n = f.ld, b = (int)nd.B.size();
       // beta = 0: the update block is written here, the children's
       // contributions to it are added afterwards (extend-add phase 1)
       add_prob(L.syrk,
-               prob(kFront, nd.foff + nd.p, n, kFront, nd.foff + nd.p, n, kFront, nd.foff + nd.p + (int64_t)nd.p * n, n,
+               prob(kFront, f.foff + f.pp, n, kFront, f.foff + f.pp, n, kFront, f.foff + f.pp + (int64_t)f.pp * n, n,
                     b, b, nd.p, -1.0, 0.0),
                true);
     }
@@ -404,19 +447,19 @@ int build_factor_plan(spde_plan* pl) {
     GemmLaunch gx, gz;
     int64_t woff = 0;
     for (const Op& o : ops[h]) {
-      const Node& nd = sym.nodes[o.node];
-      const int n = nd.n(), p = nd.p;
-      const int r = o.b - o.m, c = o.m - o.a;
+      const FrontLay& f = pl->lay[o.node];
+      const int n = f.ld, p = f.pp;
+      const int r = o.b - o.m, c = o.m - o.a, rl = (r + 15) / 16 * 16;
       // X = L_ma Z_aa (Z_aa lower), Z_ma = -Z_mm X (Z_mm lower)
-      add_prob(gx, tri(prob(kFront, nd.foff + o.m + (int64_t)o.a * n, n, kZ, nd.zoff + o.a + (int64_t)o.a * p, p,
-                            kWork, woff, r, r, c, c, 1.0, 0.0),
+      add_prob(gx, tri(prob(kFront, f.foff + o.m + (int64_t)o.a * n, n, kZ, f.zoff + o.a + (int64_t)o.a * p, p,
+                            kWork, woff, rl, r, c, c, 1.0, 0.0),
                        1),
                false, 0.5);
-      add_prob(gz, tri(prob(kZ, nd.zoff + o.m + (int64_t)o.m * p, p, kWork, woff, r, kZ,
-                            nd.zoff + o.m + (int64_t)o.a * p, p, r, c, r, -1.0, 0.0),
+      add_prob(gz, tri(prob(kZ, f.zoff + o.m + (int64_t)o.m * p, p, kWork, woff, rl, kZ,
+                            f.zoff + o.m + (int64_t)o.a * p, p, r, c, r, -1.0, 0.0),
                        3),
                false, 0.5);
-      woff += (int64_t)r * c;
+      woff += (int64_t)rl * c;
     }
     work = std::max(work, woff);
     int rc = finalize(gx, &pl->split_fs);
@@ -430,7 +473,7 @@ int build_factor_plan(spde_plan* pl) {
   // selected-inverse workspace: per level sum of b*p
   for (auto& lv : sym.levels) {
     int64_t w = 0;
-    for (int id : lv) w += (int64_t)sym.nodes[id].B.size() * sym.nodes[id].p;
+    for (int id : lv) w += (int64_t)sym.nodes[id].B.size() * pl->lay[id].pp;
     work = std::max(work, w);
   }
   work = std::max<int64_t>(work, pl->lat.Ns() * 60);
@@ -447,8 +490,8 @@ int build_factor_plan(spde_plan* pl) {
     if (rc) return rc;
     for (int c = 0; c < 2; ++c)
       for (const ExtAddDesc& d : L.h_ext[c])
-        if (d.cfoff + (int64_t)d.cld * d.cld > pl->sym.front_doubles ||
-            d.pfoff + (int64_t)d.pld * d.pld > pl->sym.front_doubles || d.cp + d.b != d.cld) {
+        if (d.cfoff + (int64_t)d.cld * (d.cp + d.b) > pl->lay_front || d.pfoff >= pl->lay_front ||
+            d.cp + d.b > d.cld) {
           set_error("extend-add descriptor out of bounds");
           return SPDE_ERR_STATE;
         }
@@ -494,12 +537,13 @@ int build_solve_plan(spde_plan* pl, int k) {
     bx.ta = true, bx.tb = false;
     for (int id : L.nodes) {
       const Node& nd = sym.nodes[id];
+      const FrontLay& f = pl->lay[id];
       const int nf = nd.n(), p = nd.p, b = (int)nd.B.size();
       const int64_t v = nd.voff * k;
-      add_prob(fy, prob(kZ, nd.zoff, p, kVec, v, nf, kX, nd.start, n, p, k, p, 1.0, 0.0), false);
-      add_prob(fu, prob(kFront, nd.foff + p, nf, kX, nd.start, n, kVec, v + p, nf, b, k, p, -1.0, 1.0), false);
-      add_prob(bt, prob(kFront, nd.foff + p, nf, kVec, v + p, nf, kVec, v, nf, p, k, b, -1.0, 1.0), false);
-      add_prob(bx, prob(kZ, nd.zoff, p, kVec, v, nf, kX, nd.start, n, p, k, p, 1.0, 0.0), false);
+      add_prob(fy, prob(kZ, f.zoff, f.pp, kVec, v, nf, kX, nd.start, n, p, k, p, 1.0, 0.0), false);
+      add_prob(fu, prob(kFront, f.foff + f.pp, f.ld, kX, nd.start, n, kVec, v + p, nf, b, k, p, -1.0, 1.0), false);
+      add_prob(bt, prob(kFront, f.foff + f.pp, f.ld, kVec, v + p, nf, kVec, v, nf, p, k, b, -1.0, 1.0), false);
+      add_prob(bx, prob(kZ, f.zoff, f.pp, kVec, v, nf, kX, nd.start, n, p, k, p, 1.0, 0.0), false);
     }
     const ArenaSizes as = arena_sizes(pl, k);
     for (GemmLaunch* g : {&fy, &fu, &bt, &bx}) {
@@ -524,31 +568,35 @@ int build_solve_plan(spde_plan* pl, int k) {
 int build_selinv_plan(spde_plan* pl) {
   const Symbolic& sym = pl->sym;
   PlanExtra* ex = extra(pl);
-  // X = L21 Z of every level keeps its own region of the workspace: the X
-  // products run ahead of the level chain on a second stream
+  // X^T = Z^T L21^T of every level keeps its own region of the workspace: the X
+  // products run ahead of the level chain on a second stream.  It is stored
+  // transposed (p x b), so that Sigma21 = -Sigma22 X reads contiguous rows of both
+  // operands and Sigma11 -= X^T Sigma21 of its first
   int64_t woff = 0;
   for (size_t l = 0; l < pl->levels.size(); ++l) {
     LevelPlan& L = pl->levels[l];
-    L.si_x.ta = false, L.si_x.tb = false;
-    L.si_s21.ta = false, L.si_s21.tb = false;
+    L.si_x.ta = true, L.si_x.tb = true;
+    L.si_s21.ta = false, L.si_s21.tb = true;
     L.si_s11a.ta = true, L.si_s11a.tb = false;
-    L.si_s11b.ta = true, L.si_s11b.tb = false;
+    L.si_s11b.ta = false, L.si_s11b.tb = false;
     std::vector<int4> gt;
     for (size_t q = 0; q < L.nodes.size(); ++q) {
       const Node& nd = sym.nodes[L.nodes[q]];
-      const int nf = nd.n(), p = nd.p, b = (int)nd.B.size();
+      const FrontLay& f = pl->lay[L.nodes[q]];
+      const int p = nd.p, b = (int)nd.B.size();
       if (b > 0 && nd.parent >= 0)
         for (int ti = 0; ti < (b + 63) / 64; ++ti)
           for (int tj = 0; tj <= ti; ++tj) gt.push_back(make_int4((int)q, ti, tj, 0));
-      add_prob(L.si_x, tri(prob(kFront, nd.foff + p, nf, kZ, nd.zoff, p, kWork, woff, b, b, p, p, 1.0, 0.0), 1), false,
-               0.5);
-      add_prob(L.si_s21, prob(kSigma, nd.foff + p + (int64_t)p * nf, nf, kWork, woff, b, kSigma, nd.foff + p, nf, b, p,
-                              b, -1.0, 0.0),
+      add_prob(L.si_x, tri(prob(kZ, f.zoff, f.pp, kFront, f.foff + f.pp, f.ld, kWork, woff, f.pp, p, b, p, 1.0, 0.0), 2),
+               false, 0.5);
+      add_prob(L.si_s21, prob(kSigma, f.foff + f.pp + (int64_t)f.pp * f.ld, f.ld, kWork, woff, f.pp, kSigma,
+                              f.foff + f.pp, f.ld, b, p, b, -1.0, 0.0),
                false);
-      add_prob(L.si_s11a, tri(prob(kZ, nd.zoff, p, kZ, nd.zoff, p, kSigma, nd.foff, nf, p, p, p, 1.0, 0.0), 2), true,
+      add_prob(L.si_s11a, tri(prob(kZ, f.zoff, f.pp, kZ, f.zoff, f.pp, kSigma, f.foff, f.ld, p, p, p, 1.0, 0.0), 2), true,
                1.0 / 3.0);
-      add_prob(L.si_s11b, prob(kWork, woff, b, kSigma, nd.foff + p, nf, kSigma, nd.foff, nf, p, p, b, -1.0, 1.0), true);
-      woff += (int64_t)b * p;
+      add_prob(L.si_s11b, prob(kWork, woff, f.pp, kSigma, f.foff + f.pp, f.ld, kSigma, f.foff, f.ld, p, p, b, -1.0, 1.0),
+               true);
+      woff += (int64_t)f.pp * b;
     }
     L.si_work = woff;
     if (woff > pl->work_doubles) {
@@ -655,8 +703,8 @@ int ensure_slot(spde_plan* pl, int slot, hipStream_t stream) {
   Slot& sl = pl->slots[slot];
   if (sl.front) return SPDE_OK;
   const Symbolic& sym = pl->sym;
-  const size_t fb = sizeof(double) * std::max<int64_t>(sym.front_doubles, 1);
-  const size_t zb = sizeof(double) * std::max<int64_t>(sym.z_doubles, 1);
+  const size_t fb = sizeof(double) * std::max<int64_t>(pl->lay_front, 1);
+  const size_t zb = sizeof(double) * std::max<int64_t>(pl->lay_z, 1);
   if (hipMalloc((void**)&sl.front, fb) != hipSuccess || hipMalloc((void**)&sl.z, zb) != hipSuccess ||
       hipMalloc((void**)&sl.work, sizeof(double) * pl->work_doubles) != hipSuccess ||
       hipMalloc((void**)&sl.partial, sizeof(double) * std::max(logdet_parts(sym.n), 1)) != hipSuccess ||
@@ -715,9 +763,7 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
     delete pl;
     return SPDE_ERR_ARG;
   }
-  const int64_t nnz = (int64_t)pl->st.indices.size();
-  pl->mapsym.resize(nnz);
-  for (int64_t e = 0; e < nnz; ++e) pl->mapsym[e] = pl->map[e] >= 0 ? pl->map[e] : pl->map[pl->st.mirror[e]];
+  build_layout(pl);
   pl->host_only = (flags & SPDE_PLAN_HOST_ONLY) != 0;
   pl->nslots = nslots;
   PlanExtra* ex = new PlanExtra();
@@ -738,6 +784,9 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
     return SPDE_OK;
   }
   const Symbolic& sym = pl->sym;
+  const std::vector<int64_t> dmap = layout_map(pl);
+  std::vector<int64_t> dmapsym(dmap.size());
+  for (size_t e = 0; e < dmap.size(); ++e) dmapsym[e] = dmap[e] >= 0 ? dmap[e] : dmap[pl->st.mirror[e]];
   int rc = SPDE_OK;
 #define TRY(x)                   \
   do {                           \
@@ -754,12 +803,12 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
   if ((int64_t)pl->st.diag.size() != sym.n) TRY((set_error("diagonal positions do not match the order"), SPDE_ERR_STATE));
   for (int64_t i = 0; i < sym.n; ++i) {
     const int64_t e = pl->st.diag[i];
-    if (e < 0 || e >= (int64_t)pl->map.size() || pl->map[e] < 0 || pl->map[e] >= sym.front_doubles)
+    if (e < 0 || e >= (int64_t)dmap.size() || dmap[e] < 0 || dmap[e] >= pl->lay_front)
       TRY((set_error("diagonal entry outside the fronts"), SPDE_ERR_STATE));
   }
   TRY(upload(&pl->d_diag, pl->st.diag));
-  TRY(upload(&pl->d_map, pl->map));
-  TRY(upload(&pl->d_mapsym, pl->mapsym));
+  TRY(upload(&pl->d_map, dmap));
+  TRY(upload(&pl->d_mapsym, dmapsym));
   TRY(upload(&pl->d_perm, sym.perm));
   std::vector<int32_t> relpos(std::max<int64_t>(sym.relpos_total, 1)), bnd(std::max<int64_t>(sym.relpos_total, 1));
   std::vector<NodeDev> nodes(sym.nodes.size());
@@ -768,10 +817,13 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
     const Node& nd = sym.nodes[q];
     for (size_t k = 0; k < nd.B.size(); ++k) {
       bnd[nd.relpos_off + k] = nd.B[k];
-      relpos[nd.relpos_off + k] = nd.relpos.empty() ? 0 : nd.relpos[k];
+      // position in the parent's padded front
+      int rp = nd.relpos.empty() ? 0 : nd.relpos[k];
+      if (nd.parent >= 0 && rp >= sym.nodes[nd.parent].p) rp += pl->lay[nd.parent].pp - sym.nodes[nd.parent].p;
+      relpos[nd.relpos_off + k] = rp;
     }
-    nodes[q] = NodeDev{nd.foff, nd.zoff, nd.voff, nd.relpos_off, nd.start, nd.p, nd.n(), nd.parent,
-                       (int32_t)nd.B.size(), nd.level, 0, 0};
+    nodes[q] = NodeDev{pl->lay[q].foff, pl->lay[q].zoff, nd.voff, nd.relpos_off, nd.start, nd.p, nd.n(), nd.parent,
+                       (int32_t)nd.B.size(), nd.level, pl->lay[q].ld, pl->lay[q].pp};
     for (int c = 0; c < nd.nchild; ++c) children[2 * q + c] = nd.child[c];
   }
   TRY(upload(&pl->d_relpos, relpos));
@@ -783,7 +835,7 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
     for (size_t q = 0; q < sym.nodes.size(); ++q) {
       // lower triangle of the own columns only (the update block is
       // written by the SYRK before anything adds to it)
-      const int nt = (sym.nodes[q].n() + 63) / 64, pt = (sym.nodes[q].p + 63) / 64;
+      const int pp = pl->lay[q].pp, nt = (pp + (int)sym.nodes[q].B.size() + 63) / 64, pt = pp / 64;
       for (int a = 0; a < nt; ++a)
         for (int b = 0; b <= a && b < pt; ++b) zt.push_back(int4{(int)q, a, b, 0});
     }
@@ -887,8 +939,8 @@ int spde_plan_get_info(const spde_plan* pl, spde_plan_info* info) {
   info->n = pl->sym.n;
   info->nnz_struct = (int64_t)pl->st.indices.size();
   info->nnz_L = pl->sym.nnz_L;
-  info->front_doubles = pl->sym.front_doubles;
-  info->z_doubles = pl->sym.z_doubles;
+  info->front_doubles = pl->lay_front;
+  info->z_doubles = pl->lay_z;
   info->nnodes = (int64_t)pl->sym.nodes.size();
   info->nlevels = (int64_t)pl->sym.levels.size();
   info->max_front = pl->sym.max_front;
@@ -1206,7 +1258,7 @@ int spde_selinv(spde_plan* pl, int slot, double* sigma, void* stream) {
   Slot& sl = pl->slots[slot];
   if (!sl.sigma) {
     SPDE_HIP(hipStreamSynchronize(s));
-    SPDE_HIP(hipMalloc((void**)&sl.sigma, sizeof(double) * std::max<int64_t>(sym.front_doubles, 1)));
+    SPDE_HIP(hipMalloc((void**)&sl.sigma, sizeof(double) * std::max<int64_t>(pl->lay_front, 1)));
   }
   if (!pl->selinv_built) {
     rc = build_selinv_plan(pl);
