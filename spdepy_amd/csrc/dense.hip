@@ -1,7 +1,6 @@
 // Dense FP64 kernels for the multifrontal factorisation, written for CDNA4
-// (gfx950): batched tile-list GEMM on v_mfma_f64_16x16x4f64 (which also does
-// the panel solve below each diagonal block, X = S W^T with W = L11^-1) and
-// the Cholesky factor + inverse of 64x64 diagonal blocks.
+// (gfx950): batched tile-list GEMM on v_mfma_f64_16x16x4f64 and the
+// bandwidth-bound products of one right-hand side.
 #include <hip/hip_runtime.h>
 
 #include "internal.hpp"
@@ -56,12 +55,9 @@ __device__ __forceinline__ void gemm_lds_body(const GemmProb* __restrict__ probs
   __shared__ double Bs[2][SB];
   const GemmTile t = tiles[SPLIT ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x)];
   const GemmProb P = probs[t.prob];
-  // A and C may be the same memory (the in-place panel solve X = S W^T,
-  // one tile column): every tile reads all of its rows of A before its
-  // epilogue writes them, and no tile reads rows another tile writes.
-  const double* A = bases.p[P.a_base] + P.a_off;
+  const double* __restrict__ A = bases.p[P.a_base] + P.a_off;
   const double* __restrict__ B = bases.p[P.b_base] + P.b_off;
-  double* C = bases.p[P.c_base] + P.c_off;
+  double* __restrict__ C = bases.p[P.c_base] + P.c_off;
   const int M = P.M, N = P.N;
   const int m0 = t.tm * BM, n0 = t.tn * BN;
   int kb = 0, K = P.K;  // this block's K range [kb, K): the zeros of a triangular operand are skipped
@@ -332,9 +328,6 @@ __device__ __forceinline__ void gemm_reg_body(const GemmProb* __restrict__ probs
         for (int v = 0; v < 4; ++v) w[(wm + y * 16 + lr) + (wn + x * 16 + lk + 4 * v) * BM] = acc[x][y][v];
     return;
   }
-  // A and C may be the same memory (the in-place panel solve, one tile
-  // column): every wave has read its rows of A before any wave writes them
-  __syncthreads();
   double* C = bases.p[P.c_base] + P.c_off;
   const double alpha = P.alpha, beta = P.beta;
   const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
@@ -540,230 +533,6 @@ void launch_gemm(const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned ld
 #undef SPDE_GEMM_FORM
 }
 
-// ------------------------------------------------ diagonal block Cholesky
-// One 256-thread block per 64x64 diagonal block.  Thread (r, g) (lane r of
-// wave g) keeps row r, columns c = 4q + g (q = 0..15), in registers, so each
-// step of four pivot columns j0..j0+3 has exactly one of them in every
-// thread.  Step: the threads publish their pivot-column entry (one LDS write
-// each, double buffered), every thread forms the 4x4 pivot block's factor
-// itself, finishes its row's four entries, writes its own one to the L copy
-// Y in LDS, and the rank-4 update of its columns right of the pivot block,
-// with the finished rows read back from Y (broadcast reads, no
-// recomputation), follows in the next step.  Entries right of the diagonal are
-// never read, so the update runs unconditionally over them.  W = L^-1 is
-// then built by recursive blocking in LDS (below).  Pivots use v_rsq_f64 with
-// two Newton steps (relative error below 2^-52) instead of a square root and
-// a division.  Blocks narrower than 64 are padded with the identity.  A
-// non-positive pivot is recorded in *status as (global elimination column
-// + 1) and replaced by 1 so the sweep completes.
-struct Piv4 {
-  double i0, i1, i2, i3, l10, l20, l30, l21, l31, l32, d0, d1, d2, d3;
-};
-
-// Keeps an updated register value where it is computed: without it the
-// compiler defers the rank-4 updates of later columns to their first use and
-// keeps every step's operands live (hundreds of registers, spilled).
-__device__ inline void pin(double& v) { asm volatile("" : "+v"(v)); }
-
-// 1/sqrt(x) for x > 0 (hardware estimate refined twice), x for the factor.
-__device__ inline double pivot_rsq(double x, bool& bad) {
-  if (!(x > 0.0)) {
-    bad = true;
-    x = 1.0;
-  }
-  double y = __builtin_amdgcn_rsq(x);
-  const double hx = 0.5 * x;
-  y = y * (1.5 - hx * y * y);
-  y = y * (1.5 - hx * y * y);
-  return y;
-}
-
-// 4x4 Cholesky factor of D(i, j) = D[i * P + j] (lower part read).
-template <int P>
-__device__ inline void chol4(const double* D, Piv4& c, int& badcol) {
-  bool b0 = false, b1 = false, b2 = false, b3 = false;
-  double x = D[0];
-  c.i0 = pivot_rsq(x, b0);
-  c.d0 = b0 ? 1.0 : x * c.i0;
-  c.l10 = D[P] * c.i0;
-  c.l20 = D[2 * P] * c.i0;
-  c.l30 = D[3 * P] * c.i0;
-  x = D[P + 1] - c.l10 * c.l10;
-  c.i1 = pivot_rsq(x, b1);
-  c.d1 = b1 ? 1.0 : x * c.i1;
-  c.l21 = (D[2 * P + 1] - c.l20 * c.l10) * c.i1;
-  c.l31 = (D[3 * P + 1] - c.l30 * c.l10) * c.i1;
-  x = D[2 * P + 2] - c.l20 * c.l20 - c.l21 * c.l21;
-  c.i2 = pivot_rsq(x, b2);
-  c.d2 = b2 ? 1.0 : x * c.i2;
-  c.l32 = (D[3 * P + 2] - c.l30 * c.l20 - c.l31 * c.l21) * c.i2;
-  x = D[3 * P + 3] - c.l30 * c.l30 - c.l31 * c.l31 - c.l32 * c.l32;
-  c.i3 = pivot_rsq(x, b3);
-  c.d3 = b3 ? 1.0 : x * c.i3;
-  badcol = b0 ? 0 : (b1 ? 1 : (b2 ? 2 : (b3 ? 3 : -1)));
-}
-
-__global__ __launch_bounds__(256) void potrf_diag_kernel(const PotrfDesc* __restrict__ descs,
-                                                         double* __restrict__ F, double* __restrict__ Z,
-                                                         int* __restrict__ status) {
-  constexpr int YP = 66;                // pitch of Y (16-byte aligned rows)
-  __shared__ double pub[2][64 * 4];     // pivot columns, row-major [r][0..3]
-  __shared__ double Y[64 * YP];         // finished L (zeros right of the diagonal)
-  __shared__ double idg[64];            // 1 / L(k, k)
-  const PotrfDesc d = descs[blockIdx.x];
-  const int tid = threadIdx.x, r = tid & 63, g = tid >> 6;
-  const int kb = d.kb;
-  double* Fb = F + d.foff + d.k0 + (int64_t)d.k0 * d.ld;
-  double a[16];
-  const int rr = r < kb ? r : kb - 1;
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int c = 4 * q + g;
-    const int cc = c < kb ? c : kb - 1;
-    const double v = Fb[rr + (int64_t)cc * d.ld];  // clamped: always inside the block
-    a[q] = (r < kb && c < kb) ? (c <= r ? v : 0.0) : (r == c ? 1.0 : 0.0);
-  }
-  // The rank-4 update of step s - 1 is applied to the next pivot column
-  // first and to the later columns during step s, beside its serial 4x4
-  // factor and row solve (same operations in the same order per entry).
-  double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const int j0 = 4 * s, buf = s & 1, jp = j0 - 4;
-    if (s > 0) {
-      const double* yc = &Y[(4 * s + g) * YP + jp];
-      a[s] -= p0 * yc[0] + p1 * yc[1] + p2 * yc[2] + p3 * yc[3];
-    }
-    pub[buf][4 * r + g] = a[s];
-    __syncthreads();
-    Piv4 c;
-    int bad;
-    chol4<4>(&pub[buf][4 * j0], c, bad);
-    if (bad >= 0 && tid == 0 && j0 + bad < kb) atomicCAS(status, 0, d.colbase + j0 + bad + 1);
-    if (s > 0) {
-#pragma unroll
-      for (int q = s + 1; q < 16; ++q) {
-        const double* yc = &Y[(4 * q + g) * YP + jp];
-        a[q] -= p0 * yc[0] + p1 * yc[1] + p2 * yc[2] + p3 * yc[3];
-      }
-    }
-    // row r's four entries; on the pivot rows this yields the factor's
-    // entries left of and on the diagonal, the rest (and all of the rows
-    // above) are cleared
-    const double* pr = &pub[buf][4 * r];
-    double y0 = pr[0] * c.i0;
-    double y1 = (pr[1] - y0 * c.l10) * c.i1;
-    double y2 = (pr[2] - y0 * c.l20 - y1 * c.l21) * c.i2;
-    double y3 = (pr[3] - y0 * c.l30 - y1 * c.l31 - y2 * c.l32) * c.i3;
-    y0 = (r >= j0) ? y0 : 0.0;
-    y1 = (r >= j0 + 1) ? y1 : 0.0;
-    y2 = (r >= j0 + 2) ? y2 : 0.0;
-    y3 = (r >= j0 + 3) ? y3 : 0.0;
-    const double mine = (g == 0) ? y0 : (g == 1 ? y1 : (g == 2 ? y2 : y3));
-    a[s] = mine;
-    Y[r * YP + j0 + g] = mine;
-    if (tid < 4) idg[j0 + tid] = (tid == 0) ? c.i0 : (tid == 1 ? c.i1 : (tid == 2 ? c.i2 : c.i3));
-    __syncthreads();
-    p0 = y0;
-    p1 = y1;
-    p2 = y2;
-    p3 = y3;
-#pragma unroll
-    for (int q = s + 1; q < 16; ++q) pin(a[q]);
-  }
-  if (r < kb) {
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int c = 4 * q + g;
-      if (c < kb && c <= r) Fb[r + (int64_t)c * d.ld] = a[q];
-    }
-  }
-  // W = L^-1 by recursive blocking: the four 16x16 diagonal blocks are
-  // inverted by column-oriented forward substitution (wave g, lane j < 16:
-  // column j of block g), then W21 = -W22 (L21 W11) for the two 32x32 and
-  // the 64x64 block rows, the products spread over the block.  Wl is
-  // row-major with zeros above the diagonal; blocks beyond kb hold the
-  // identity padding of L, so W is the identity there too.
-  constexpr int WP = 65;
-  __shared__ double Wl[64 * WP];
-  __shared__ double Xs[32 * 33];
-  for (int e = tid; e < 64 * WP; e += 256) Wl[e] = 0.0;
-  __syncthreads();
-  if (r < 16) {
-    const int o = 16 * g, j = r;
-    double x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = (i == j) ? 1.0 : 0.0;
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      x[kk] *= idg[o + kk];
-#pragma unroll
-      for (int i = kk + 1; i < 16; ++i) x[i] -= Y[(o + i) * YP + o + kk] * x[kk];
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) Wl[(o + i) * WP + o + j] = x[i];
-  }
-  __syncthreads();
-  {
-    // 32 level, pair P = rows/cols 32P .. 32P + 31: X = L(o+16.., o..) W00,
-    // W10 = -W11 X; thread: pair tid >> 7, row i, columns j0, j0 + 1
-    const int P = tid >> 7, t = tid & 127, i = t >> 3, j0 = (t & 7) * 2, o = 32 * P;
-    double x0 = 0.0, x1 = 0.0;
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const double l = Y[(o + 16 + i) * YP + o + kk];
-      x0 += l * Wl[(o + kk) * WP + o + j0];
-      x1 += l * Wl[(o + kk) * WP + o + j0 + 1];
-    }
-    Xs[(P * 16 + i) * 33 + j0] = x0;
-    Xs[(P * 16 + i) * 33 + j0 + 1] = x1;
-    __syncthreads();
-    double w0 = 0.0, w1 = 0.0;
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const double v = Wl[(o + 16 + i) * WP + o + 16 + kk];
-      w0 += v * Xs[(P * 16 + kk) * 33 + j0];
-      w1 += v * Xs[(P * 16 + kk) * 33 + j0 + 1];
-    }
-    Wl[(o + 16 + i) * WP + o + j0] = -w0;
-    Wl[(o + 16 + i) * WP + o + j0 + 1] = -w1;
-  }
-  __syncthreads();
-  {
-    // 64 level: X = L(32.., 0..31) W_aa, W_ba = -W_bb X; thread: column
-    // j = tid & 31, rows i0 + 8u
-    const int j = tid & 31, i0 = tid >> 5;
-    double x[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int kk = 0; kk < 32; ++kk) {
-      const double wv = Wl[kk * WP + j];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) x[u] += Y[(32 + i0 + 8 * u) * YP + kk] * wv;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) Xs[(i0 + 8 * u) * 33 + j] = x[u];
-    __syncthreads();
-    double w[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int kk = 0; kk < 32; ++kk) {
-      const double xv = Xs[kk * 33 + j];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) w[u] += Wl[(32 + i0 + 8 * u) * WP + 32 + kk] * xv;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) Wl[(32 + i0 + 8 * u) * WP + j] = -w[u];
-  }
-  __syncthreads();
-  double* Zb = Z + d.zoff + d.k0 + (int64_t)d.k0 * d.zld;
-  if (r < kb) {
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int c = 4 * q + g;
-      if (c < kb) Zb[r + (int64_t)c * d.zld] = Wl[r * WP + c];
-    }
-  }
-}
-
 __global__ void fill_kernel(double* __restrict__ p, int64_t n, double v) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     p[i] = v;
@@ -784,9 +553,6 @@ __global__ __launch_bounds__(64) void mfma_probe_kernel(int which, double* __res
   for (int v = 0; v < 4; ++v) out[4 * l + v] = acc[v];
 }
 
-void launch_potrf(const PotrfDesc* d, int n, double* F, double* Z, int* status, hipStream_t s) {
-  if (n > 0) hipLaunchKernelGGL(potrf_diag_kernel, dim3(n), dim3(256), 0, s, d, F, Z, status);
-}
 void launch_fill(double* p, int64_t n, double v, hipStream_t s) {
   if (n <= 0) return;
   int64_t blocks = (n + 255) / 256;

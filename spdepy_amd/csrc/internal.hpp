@@ -78,12 +78,16 @@ struct GemmLaunch {
 // against 3.8 and 10.6 ms with the per-column kernel).
 constexpr int kGemvMaxN = 1;
 
-struct PotrfDesc {      // one diagonal block of one front
-  int64_t foff;         // front offset
-  int64_t zoff;         // Z offset of the block's node
-  int32_t ld, zld;      // front dimension, p
-  int32_t k0, kb;       // block start (within own columns) and width
-  int32_t node, colbase;
+struct FrontDesc {      // one front of a level's factorisation
+  int64_t foff, zoff;
+  int32_t ld, pp, p, nrows;  // nrows = pp + boundary rows
+  int32_t R, P;         // row tiles and own column tiles of 64
+  int32_t flag0;        // counter of tile (i, k): flag0 + k R + i
+  int32_t colbase;      // elimination column of the first own column
+};
+constexpr int kStalled = -1;  // status of a factorisation whose waits gave up
+struct FrontTask {      // i = j: the diagonal block j; else tiles (i, j), (i + 1, j)
+  int32_t front, j, i, pad;
 };
 struct ExtAddDesc {     // extend-add of a child's update block into its parent
   int64_t cfoff, pfoff, relpos_off;
@@ -92,13 +96,6 @@ struct ExtAddDesc {     // extend-add of a child's update block into its parent
 };
 struct ExtAddTile {
   int32_t desc, ti, tj, phase;  // phase 0: columns < split, 1: columns >= split
-};
-
-struct Step {           // one stage of the dense partial factorisation of a level
-  int npotrf = 0;
-  PotrfDesc* d_potrf = nullptr;
-  GemmLaunch panel;     // rows below the diagonal blocks: X = S W^T, in place
-  GemmLaunch update;    // trailing update of the nodes' own columns
 };
 
 struct LevelPlan {
@@ -111,22 +108,25 @@ struct LevelPlan {
   ExtAddTile* d_exttile[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
   std::vector<ExtAddDesc> h_ext[2];
   std::vector<ExtAddTile> h_exttile[2][2];
-  std::vector<Step> steps;
+  // factorisation of the own columns: fronts and tasks in ticket order
+  FrontDesc* d_fronts = nullptr;
+  FrontTask* d_tasks = nullptr;
+  int ntasks = 0;
   GemmLaunch syrk;
   // solves / selinv
   GemmLaunch fwd_y, fwd_u, bwd_t, bwd_x;   // the current nrhs' launches (owned by solve_cache)
   GemmLaunch si_x, si_s21, si_s11a, si_s11b;
-  int64_t si_work = 0;
 };
 
 struct Slot {
   double* front = nullptr;  // factor fronts
   double* z = nullptr;      // inverses of the diagonal blocks of L
   double* sigma = nullptr;  // selected-inverse fronts (allocated on first use)
-  double* work = nullptr;   // inverse-of-L11 and selected-inverse temporaries
+  double* work = nullptr;   // inverse-of-L11 temporaries
   double* partial = nullptr;  // log-det partial sums per 256 variables
   double* ld = nullptr;     // device log-det
   int* status = nullptr;    // first non-positive pivot (elimination column + 1)
+  int* flags = nullptr;     // factorisation: stop flag, a ticket counter per level, tile counters
   double* vec = nullptr;    // solve front vectors
   int64_t vec_cap = 0;      // in doubles
   double* xy = nullptr;     // elimination-ordered solve buffer
@@ -193,6 +193,7 @@ struct spde_plan {
   int32_t* d_spcol = nullptr;
   int64_t work_doubles = 0;       // per-slot workspace size
   std::vector<spde::FrontLay> lay;  // device layout per node
+  int nflags = 0;                   // tile counters of the factorisation (all levels)
   int64_t lay_front = 0, lay_z = 0;  // arena sizes (doubles) of that layout
   std::vector<spde::Slot> slots;
   std::vector<spde::LevelPlan> levels;

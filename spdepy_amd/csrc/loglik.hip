@@ -336,6 +336,10 @@ int spde_loglik_finish(spde_plan* pl, spde_loglik_out* out) {
   for (int q = 0; q < 3; ++q)
     if (st[q] != 0) {
       owner[q]->slots[slot[q]].factored = false;
+      if (st[q] == kStalled) {
+        set_error("spde_loglik: a factorisation stalled");
+        return SPDE_ERR_HIP;
+      }
       set_error(std::string("spde_loglik: ") + (q == 0 ? "Q_c" : (q == 1 ? "Q0" : "B^T B")) +
                 " is not positive definite (pivot at lattice index " +
                 std::to_string(owner[q]->sym.perm[st[q] - 1]) + ")");

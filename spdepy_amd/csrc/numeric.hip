@@ -14,7 +14,9 @@
 namespace spde {
 
 void launch_gemm(const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned lds = 0);
-void launch_potrf(const PotrfDesc* d, int n, double* F, double* Z, int* status, hipStream_t s);
+void launch_front_factor(const FrontDesc* fronts, const FrontTask* tasks, int ntasks, double* F, double* Z, int* flags,
+                         int* ticket, int* stop, int* status, hipStream_t s);
+void launch_clear_flags(int* p, int n, hipStream_t s);
 void launch_fill(double* p, int64_t n, double v, hipStream_t s);
 void launch_scatter(const double* q, const int64_t* map, int64_t nnz, double* F, hipStream_t s);
 void launch_diag_add(const double* add, const int64_t* diag, const int64_t* map, int64_t n, double* F, hipStream_t s);
@@ -306,6 +308,88 @@ GemmProb prob(int8_t ab, int64_t ao, int lda, int8_t bb, int64_t bo, int ldb, in
   return P;
 }
 
+// Fronts and tasks of one level in ticket order: by column j over all fronts,
+// diagonal j, then diagonal j + 1 ahead of the tiles below j (it waits for W_j
+// only), then those tiles, two row tiles to a task.  Checked here: every tile
+// that a task waits for is produced by a task with a lower ticket.
+int build_front_tasks(spde_plan* pl, LevelPlan& L) {
+  const Symbolic& sym = pl->sym;
+  std::vector<FrontDesc> fd;
+  int pmax = 0;
+  for (int id : L.nodes) {
+    const Node& nd = sym.nodes[id];
+    const FrontLay& f = pl->lay[id];
+    if (nd.p == 0) continue;
+    FrontDesc d{};
+    d.foff = f.foff;
+    d.zoff = f.zoff;
+    d.ld = f.ld;
+    d.pp = f.pp;
+    d.p = nd.p;
+    d.nrows = f.pp + (int)nd.B.size();
+    d.R = (d.nrows + 63) / 64;
+    d.P = f.pp / 64;
+    d.flag0 = pl->nflags;
+    d.colbase = nd.start;
+    if (f.pp != 64 * ((nd.p + 63) / 64) || f.foff + (int64_t)f.ld * d.nrows > pl->lay_front || f.ld < d.nrows ||
+        f.zoff + (int64_t)f.pp * f.pp > pl->lay_z || (f.foff & 15) || (f.ld & 15) || (f.zoff & 15)) {
+      set_error("front layout out of bounds");
+      return SPDE_ERR_STATE;
+    }
+    pl->nflags += d.R * d.P;
+    pmax = std::max(pmax, d.P);
+    fd.push_back(d);
+  }
+  std::vector<FrontTask> tasks;
+  for (size_t q = 0; q < fd.size(); ++q) tasks.push_back({(int32_t)q, 0, 0, 0});
+  for (int j = 0; j < pmax; ++j) {
+    for (size_t q = 0; q < fd.size(); ++q)
+      if (j + 1 < fd[q].P) tasks.push_back({(int32_t)q, j + 1, j + 1, 0});
+    for (size_t q = 0; q < fd.size(); ++q) {
+      if (j >= fd[q].P) continue;
+      for (int i = j + 1 < fd[q].P ? j + 2 : j + 1; i < fd[q].R; i += 2) tasks.push_back({(int32_t)q, j, i, 0});
+    }
+  }
+  std::vector<std::vector<int>> made(fd.size());  // ticket of each tile
+  for (size_t q = 0; q < fd.size(); ++q) made[q].assign((size_t)fd[q].R * fd[q].P, -1);
+  auto at = [&](int q, int i, int k) -> int& { return made[q][(size_t)k * fd[q].R + i]; };
+  for (size_t t = 0; t < tasks.size(); ++t) {
+    const FrontTask& T = tasks[t];
+    if (T.i == T.j) {
+      at(T.front, T.j, T.j) = (int)t;
+      if (T.j > 0) at(T.front, T.j, T.j - 1) = (int)t;
+    } else {
+      for (int i = T.i; i < std::min(T.i + 2, fd[T.front].R); ++i) at(T.front, i, T.j) = (int)t;
+    }
+  }
+  bool ok = true;
+  for (size_t t = 0; t < tasks.size(); ++t) {
+    const FrontTask& T = tasks[t];
+    auto before = [&](int i, int k) {
+      const int m = at(T.front, i, k);
+      ok = ok && m >= 0 && m < (int)t;
+    };
+    if (T.i == T.j) {
+      for (int k = 0; k + 1 < T.j; ++k) before(T.j, k), before(T.j - 1, k);
+      if (T.j > 0) before(T.j - 1, T.j - 1);
+    } else {
+      for (int k = 0; k < T.j; ++k) {
+        before(T.j, k);
+        for (int i = T.i; i < std::min(T.i + 2, fd[T.front].R); ++i) before(i, k);
+      }
+      before(T.j, T.j);
+    }
+  }
+  if (!ok) {
+    set_error("factorisation tasks out of order");
+    return SPDE_ERR_STATE;
+  }
+  L.ntasks = (int)tasks.size();
+  int rc = upload(&L.d_fronts, fd);
+  if (rc) return rc;
+  return upload(&L.d_tasks, tasks);
+}
+
 int build_factor_plan(spde_plan* pl) {
   const Symbolic& sym = pl->sym;
   pl->split_fs = 0;
@@ -340,74 +424,8 @@ int build_factor_plan(spde_plan* pl) {
         if (rc) return rc;
       }
     }
-    int pmax = 0;
-    for (int id : L.nodes) pmax = std::max(pmax, sym.nodes[id].p);
-    // Recursive column blocking of the nodes' own columns: rec(a, b) factors
-    // columns [a, b) as rec(a, m), one update of columns [m, b) (all rows
-    // below m) by columns [a, m) with depth m - a, rec(m, b); leaves are
-    // 64-column steps (diagonal-block Cholesky + panel solve).  Same flops
-    // as the right-looking sweep, but the trailing updates are few and deep
-    // instead of one depth-64 pass over the trailing matrix per step.
-    std::function<int(int, int)> rec = [&](int a, int b) -> int {
-      Step st;
-      st.panel.ta = false;
-      st.panel.tb = true;
-      st.update.ta = false;
-      st.update.tb = true;
-      if (b - a <= NB) {
-        const int k0 = a;
-        std::vector<PotrfDesc> pd;
-        for (int id : L.nodes) {
-          const Node& nd = sym.nodes[id];
-          if (nd.p <= k0) continue;
-          const FrontLay& f = pl->lay[id];
-          const int n = f.ld, kb = std::min(NB, nd.p - k0);
-          pd.push_back({f.foff, f.zoff, n, f.pp, k0, kb, id, nd.start + k0});
-          // rows below the block: the own rows, then (past the padding) the boundary
-          const int r0 = k0 + kb < nd.p ? k0 + kb : f.pp;
-          const int M = f.pp + (int)nd.B.size() - r0;
-          const int64_t off = f.foff + r0 + (int64_t)k0 * n;
-          // in place (kb <= 64: one tile column); W is lower triangular
-          add_prob(st.panel,
-                   prob(kFront, off, n, kZ, f.zoff + k0 + (int64_t)k0 * f.pp, f.pp, kFront, off, n, M, kb, kb, 1.0, 0.0),
-                   false, 0.5);
-        }
-        st.npotrf = (int)pd.size();
-        int rc = upload(&st.d_potrf, pd);
-        if (rc) return rc;
-        rc = finalize(st.panel, &pl->split_fs);
-        if (rc) return rc;
-        for (const GemmProb& P : st.panel.h_probs)
-          if (P.N > st.panel.tile) {  // the in-place solve needs one tile column
-            set_error("panel solve wider than a tile");
-            return SPDE_ERR_STATE;
-          }
-        L.steps.push_back(std::move(st));
-        return SPDE_OK;
-      }
-      int half = (b - a + 1) / 2;
-      half = ((half + NB - 1) / NB) * NB;
-      const int m = a + half;
-      int rc = rec(a, m);
-      if (rc) return rc;
-      for (int id : L.nodes) {
-        const Node& nd = sym.nodes[id];
-        if (nd.p <= m) continue;
-        const FrontLay& f = pl->lay[id];
-        const int n = f.ld, M = f.pp + (int)nd.B.size() - m, N = std::min(b, nd.p) - m, K = m - a;
-        const int64_t ab = f.foff + m + (int64_t)a * n;
-        add_prob(st.update, prob(kFront, ab, n, kFront, ab, n, kFront, f.foff + m + (int64_t)m * n, n, M, N, K, -1.0, 1.0),
-                 true);
-      }
-      rc = finalize(st.update, &pl->split_fs);
-      if (rc) return rc;
-      L.steps.push_back(std::move(st));
-      return rec(m, b);
-    };
-    if (pmax > 0) {
-      int rc = rec(0, pmax);
-      if (rc) return rc;
-    }
+    int rcf = build_front_tasks(pl, L);
+    if (rcf) return rcf;
     L.syrk.ta = false;
     L.syrk.tb = true;
     for (int id : L.nodes) {
@@ -470,22 +488,10 @@ int build_factor_plan(spde_plan* pl) {
     pl->trtri.push_back(std::move(gz));
   }
   pl->trtri_heights = (int)(pl->trtri.size() / 2);
-  // selected-inverse workspace: per level sum of b*p
-  for (auto& lv : sym.levels) {
-    int64_t w = 0;
-    for (int id : lv) w += (int64_t)sym.nodes[id].B.size() * pl->lay[id].pp;
-    work = std::max(work, w);
-  }
   work = std::max<int64_t>(work, pl->lat.Ns() * 60);
   pl->work_doubles = std::max<int64_t>(work, 1);
   const ArenaSizes as = arena_sizes(pl, 1);
   for (auto& L : pl->levels) {
-    for (auto& st : L.steps) {
-      int rc = validate(st.panel, as, "factor panel");
-      if (rc) return rc;
-      rc = validate(st.update, as, "factor update");
-      if (rc) return rc;
-    }
     int rc = validate(L.syrk, as, "factor syrk");
     if (rc) return rc;
     for (int c = 0; c < 2; ++c)
@@ -568,11 +574,11 @@ int build_solve_plan(spde_plan* pl, int k) {
 int build_selinv_plan(spde_plan* pl) {
   const Symbolic& sym = pl->sym;
   PlanExtra* ex = extra(pl);
-  // X^T = Z^T L21^T of every level keeps its own region of the workspace: the X
-  // products run ahead of the level chain on a second stream.  It is stored
-  // transposed (p x b), so that Sigma21 = -Sigma22 X reads contiguous rows of both
-  // operands and Sigma11 -= X^T Sigma21 of its first
-  int64_t woff = 0;
+  // X^T = Z^T L21^T (p x b) lives in its front's own block right of the own
+  // columns (rows [0, p), columns from pp), which the selected inverse does not
+  // use otherwise: the X products run ahead of the level chain on a second stream
+  // without a workspace.  Stored transposed, Sigma21 = -Sigma22 X reads contiguous
+  // rows of both operands and Sigma11 -= X^T Sigma21 of its first
   for (size_t l = 0; l < pl->levels.size(); ++l) {
     LevelPlan& L = pl->levels[l];
     L.si_x.ta = true, L.si_x.tb = true;
@@ -587,24 +593,15 @@ int build_selinv_plan(spde_plan* pl) {
       if (b > 0 && nd.parent >= 0)
         for (int ti = 0; ti < (b + 63) / 64; ++ti)
           for (int tj = 0; tj <= ti; ++tj) gt.push_back(make_int4((int)q, ti, tj, 0));
-      add_prob(L.si_x, tri(prob(kZ, f.zoff, f.pp, kFront, f.foff + f.pp, f.ld, kWork, woff, f.pp, p, b, p, 1.0, 0.0), 2),
+      const int64_t xo = f.foff + (int64_t)f.pp * f.ld;
+      add_prob(L.si_x, tri(prob(kZ, f.zoff, f.pp, kFront, f.foff + f.pp, f.ld, kSigma, xo, f.ld, p, b, p, 1.0, 0.0), 2),
                false, 0.5);
-      add_prob(L.si_s21, prob(kSigma, f.foff + f.pp + (int64_t)f.pp * f.ld, f.ld, kWork, woff, f.pp, kSigma,
-                              f.foff + f.pp, f.ld, b, p, b, -1.0, 0.0),
+      add_prob(L.si_s21, prob(kSigma, xo + f.pp, f.ld, kSigma, xo, f.ld, kSigma, f.foff + f.pp, f.ld, b, p, b, -1.0, 0.0),
                false);
       add_prob(L.si_s11a, tri(prob(kZ, f.zoff, f.pp, kZ, f.zoff, f.pp, kSigma, f.foff, f.ld, p, p, p, 1.0, 0.0), 2), true,
                1.0 / 3.0);
-      add_prob(L.si_s11b, prob(kWork, woff, f.pp, kSigma, f.foff + f.pp, f.ld, kSigma, f.foff, f.ld, p, p, b, -1.0, 1.0),
+      add_prob(L.si_s11b, prob(kSigma, xo, f.ld, kSigma, f.foff + f.pp, f.ld, kSigma, f.foff, f.ld, p, p, b, -1.0, 1.0),
                true);
-      woff += (int64_t)f.pp * b;
-    }
-    L.si_work = woff;
-    if (woff > pl->work_doubles) {
-      if (!pl->slots.empty()) {  // the slots' workspaces are allocated after this plan is built
-        set_error("selected-inverse workspace too small");
-        return SPDE_ERR_STATE;
-      }
-      pl->work_doubles = woff;
     }
     const ArenaSizes as = arena_sizes(pl, 1);
     for (GemmLaunch* g : {&L.si_x, &L.si_s21, &L.si_s11a, &L.si_s11b}) {
@@ -695,6 +692,9 @@ Bases make_bases(spde_plan* pl, int slot, double* x) {
   return b;
 }
 
+// Words of a slot's factorisation counters: stop flag, tickets, tiles.
+int flag_words(const spde_plan* pl) { return 1 + (int)pl->levels.size() + pl->nflags; }
+
 // Device arenas of a factor slot, allocated on its first factorisation.  The
 // fronts and Z are cleared once (on the factorisation's stream): later
 // factorisations clear only the lower triangles, and nothing writes above a
@@ -709,11 +709,13 @@ int ensure_slot(spde_plan* pl, int slot, hipStream_t stream) {
       hipMalloc((void**)&sl.work, sizeof(double) * pl->work_doubles) != hipSuccess ||
       hipMalloc((void**)&sl.partial, sizeof(double) * std::max(logdet_parts(sym.n), 1)) != hipSuccess ||
       hipMalloc((void**)&sl.ld, sizeof(double)) != hipSuccess ||
+      hipMalloc((void**)&sl.flags, sizeof(int) * flag_words(pl)) != hipSuccess ||
       hipMalloc((void**)&sl.status, sizeof(int)) != hipSuccess) {
-    for (void* p : {(void*)sl.front, (void*)sl.z, (void*)sl.work, (void*)sl.partial, (void*)sl.ld, (void*)sl.status})
+    for (void* p : {(void*)sl.front, (void*)sl.z, (void*)sl.work, (void*)sl.partial, (void*)sl.ld, (void*)sl.status,
+                    (void*)sl.flags})
       if (p) hipFree(p);
     sl.front = sl.z = sl.work = sl.partial = sl.ld = nullptr;
-    sl.status = nullptr;
+    sl.status = sl.flags = nullptr;
     set_error("factor slot " + std::to_string(slot) + ": device allocation of " +
               std::to_string((fb + zb) >> 20) + " MiB failed");
     return SPDE_ERR_ALLOC;
@@ -893,6 +895,7 @@ void spde_plan_destroy(spde_plan* pl) {
       hipFree(s.partial);
       hipFree(s.ld);
       hipFree(s.status);
+      hipFree(s.flags);
       hipFree(s.vec);
       hipFree(s.xy);
       hipFree(s.splitws);
@@ -903,11 +906,8 @@ void spde_plan_destroy(spde_plan* pl) {
         hipFree(L.d_exttile[0][s]);
         hipFree(L.d_exttile[1][s]);
       }
-      for (auto& st : L.steps) {
-        hipFree(st.d_potrf);
-        free_launch(st.panel);
-        free_launch(st.update);
-      }
+      hipFree(L.d_fronts);
+      hipFree(L.d_tasks);
       for (GemmLaunch* g : {&L.syrk, &L.si_x, &L.si_s21, &L.si_s11a, &L.si_s11b}) free_launch(*g);
     }
     for (auto& g : pl->trtri) free_launch(g);
@@ -1002,6 +1002,7 @@ int spde_factor_async(spde_plan* pl, int slot, const double* qval, const double*
   rc = ensure_splitws(pl, slot);
   if (rc) return rc;
   hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(64), 0, s, sl.status);
+  launch_clear_flags(sl.flags, flag_words(pl), s);
   launch_zero_lower(pl->d_nodes, ex->d_ztiles, ex->nztiles, sl.front, s);
   launch_scatter(qval, pl->d_map, (int64_t)pl->st.indices.size(), sl.front, s);
   if (diag_add) launch_diag_add(diag_add, pl->d_diag, pl->d_map, sym.n, sl.front, s);
@@ -1009,11 +1010,8 @@ int spde_factor_async(spde_plan* pl, int slot, const double* qval, const double*
   for (size_t l = 0; l < pl->levels.size(); ++l) {
     LevelPlan& L = pl->levels[l];
     for (int c = 0; c < 2; ++c) launch_extend_add(L.d_ext[c], L.d_exttile[0][c], L.next[0][c], pl->d_relpos, sl.front, s);
-    for (Step& st : L.steps) {  // a leaf (potrf + panel) or an update
-      launch_potrf(st.d_potrf, st.npotrf, sl.front, sl.z, sl.status, s);
-      run_gemm(pl, st.panel, b, s);
-      run_gemm(pl, st.update, b, s);
-    }
+    launch_front_factor(L.d_fronts, L.d_tasks, L.ntasks, sl.front, sl.z, sl.flags + 1 + pl->levels.size(),
+                        sl.flags + 1 + l, sl.flags, sl.status, s);
     run_gemm(pl, L.syrk, b, s);
     for (int c = 0; c < 2; ++c) launch_extend_add(L.d_ext[c], L.d_exttile[1][c], L.next[1][c], pl->d_relpos, sl.front, s);
   }
@@ -1040,6 +1038,10 @@ int spde_factor_finish(spde_plan* pl, int slot, double* logdet) {
   SPDE_HIP(hipStreamSynchronize(sl.stream));
   if (status != 0) {
     sl.factored = false;
+    if (status == kStalled) {
+      set_error("spde_factor: the factorisation stalled");
+      return SPDE_ERR_HIP;
+    }
     const int col = status - 1;
     set_error("spde_factor: matrix is not positive definite (pivot at lattice index " +
               std::to_string(pl->sym.perm[col]) + ")");
