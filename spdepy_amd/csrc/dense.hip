@@ -231,7 +231,9 @@ __device__ __forceinline__ void load_tail(double (&f)[T][4], const uint32_t (&of
   }
 }
 
-template <bool TA, bool TB, bool VEC, int TM, int TN, bool SPLIT = false>
+// PULL: C = alpha op(A) op(B) + the children's update blocks (the extend-add
+// of the multifrontal method, read once in place of a read-modify-write of C).
+template <bool TA, bool TB, bool VEC, int TM, int TN, bool SPLIT = false, bool PULL = false>
 __device__ __forceinline__ void gemm_reg_body(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles,
                                               const Bases& bases, int split = 1, double* __restrict__ ws = nullptr) {
   constexpr int BM = 32 * TM, BN = 32 * TN;  // four waves, 2 x 2
@@ -334,20 +336,39 @@ __device__ __forceinline__ void gemm_reg_body(const GemmProb* __restrict__ probs
   // lower problems: the part of a tile above the diagonal is left
   // untouched (it is never read, and stays as initialised)
   const bool straddles = P.lower && m0 < n0 + BN;
-#pragma unroll
-  for (int x = 0; x < TN; ++x)
+  Pull q{};
+  int im[TM][2];
+  if constexpr (PULL) {
+    q = bases.pulls[P.pull];
 #pragma unroll
     for (int y = 0; y < TM; ++y)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
+      for (int c = 0; c < 2; ++c)
+        im[y][c] = child_row(bases.inv, q, c, P.pull_row + min(m0 + wm + y * 16 + lr, M - 1));
+  }
+#pragma unroll
+  for (int x = 0; x < TN; ++x)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int n = n0 + wn + x * 16 + lk + 4 * v;
+      int jn[2];
+      if constexpr (PULL) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) jn[c] = child_row(bases.inv, q, c, P.pull_row + min(n, N - 1));
+      }
+#pragma unroll
+      for (int y = 0; y < TM; ++y) {
         const int m = m0 + wm + y * 16 + lr;
-        const int n = n0 + wn + x * 16 + lk + 4 * v;
         if ((interior || (m < M && n < N)) && !(straddles && m < n)) {
           double* c = C + m + (int64_t)n * P.ldc;
           const double r = alpha * acc[x][y][v];
-          *c = (beta == 0.0) ? r : r + beta * (*c);
+          if constexpr (PULL)
+            *c = assembled(bases.p[kFront], r, q, im[y][0], im[y][1], jn[0], jn[1]);
+          else
+            *c = (beta == 0.0) ? r : r + beta * (*c);
         }
       }
+    }
 }
 
 // 64x64 tiles.
@@ -358,6 +379,13 @@ __global__ __launch_bounds__(256) void gemm64_kernel(const GemmProb* __restrict_
     gemm_lds_body<TA, TB, 64, 64>(probs, tiles, bases);
   else
     gemm_reg_body<TA, TB, VEC, 2, 2>(probs, tiles, bases);
+}
+
+// The level SYRK with the children's update blocks.
+template <int TM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TM == 4 ? 3 : 4, TM == 4 ? 3 : 8))) void
+syrk_pull_kernel(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles, Bases bases) {
+  gemm_reg_body<false, true, true, TM, 2, false, true>(probs, tiles, bases);
 }
 
 // Split-K partial tiles (64x64) and their ordered sum.
@@ -371,9 +399,11 @@ __global__ __launch_bounds__(256) void gemm64_split_kernel(const GemmProb* __res
     gemm_reg_body<TA, TB, VEC, 2, 2, true>(probs, tiles, bases, split, ws);
 }
 
+// PULL: plus the children's update blocks (beta not used).
 // Block b: C tile of tiles[b * split] = alpha * sum_q partial[b * split + q]
 // (q ascending) + beta C, inside the problem and, for lower problems, on or
 // below the diagonal.
+template <bool PULL>
 __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmProb* __restrict__ probs,
                                                            const GemmTile* __restrict__ tiles, Bases bases, int split,
                                                            const double* __restrict__ ws) {
@@ -390,7 +420,14 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmProb* __res
     for (int q = 0; q < split; ++q) acc += w[(int64_t)q * 4096 + e];
     double* c = C + m + (int64_t)n * P.ldc;
     const double r = P.alpha * acc;
-    *c = (P.beta == 0.0) ? r : r + P.beta * (*c);
+    if constexpr (PULL) {
+      const Pull pq = bases.pulls[P.pull];
+      const int i = P.pull_row + m, j = P.pull_row + n;
+      *c = assembled(bases.p[kFront], r, pq, child_row(bases.inv, pq, 0, i), child_row(bases.inv, pq, 1, i),
+                     child_row(bases.inv, pq, 0, j), child_row(bases.inv, pq, 1, j));
+    } else {
+      *c = (P.beta == 0.0) ? r : r + P.beta * (*c);
+    }
   }
 }
 
@@ -522,8 +559,19 @@ void launch_gemm(const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned ld
   if (g.split > 1) {
     double* ws = b.ws + g.ws_off;
     SPDE_GEMM_FORM(gemm64_split_kernel, grid, block, 0, s, g.d_probs, g.d_tiles, b, g.split, ws);
-    hipLaunchKernelGGL(split_reduce_kernel, dim3(g.ntiles / g.split), block, 0, s, g.d_probs, g.d_tiles, b, g.split,
-                       ws);
+    if (g.pull)
+      hipLaunchKernelGGL(split_reduce_kernel<true>, dim3(g.ntiles / g.split), block, 0, s, g.d_probs, g.d_tiles, b,
+                         g.split, ws);
+    else
+      hipLaunchKernelGGL(split_reduce_kernel<false>, dim3(g.ntiles / g.split), block, 0, s, g.d_probs, g.d_tiles, b,
+                         g.split, ws);
+    return;
+  }
+  if (g.pull) {
+    if (g.tile == 128)
+      hipLaunchKernelGGL(syrk_pull_kernel<4>, grid, block, lds, s, g.d_probs, g.d_tiles, b);
+    else
+      hipLaunchKernelGGL(syrk_pull_kernel<2>, grid, block, lds, s, g.d_probs, g.d_tiles, b);
     return;
   }
   if (g.tile == 128)
@@ -613,6 +661,9 @@ extern "C" int spde_debug_gemm(int ta, int tb, int M, int N, int K, double alpha
   bs.p[0] = const_cast<double*>(A);
   bs.p[1] = const_cast<double*>(B);
   bs.p[2] = C;
+  bs.ws = nullptr;
+  bs.pulls = nullptr;
+  bs.inv = nullptr;
   launch_gemm(g, bs, (hipStream_t)stream, 0);
   SPDE_HIP(hipStreamSynchronize((hipStream_t)stream));
   hipFree(g.d_probs);

@@ -28,9 +28,32 @@ constexpr int kTmpl = 143;  // per-cell assembly template (doubles)
 
 // Operand base pointers of a batched launch (selected per operand by id).
 enum Base : int8_t { kFront = 0, kZ = 1, kSigma = 2, kWork = 3, kVec = 4, kX = 5, kNumBases = 6 };
+// Update blocks of a front's children, read where the front's entries are
+// formed: u: offset of child s's update block, inv + i: row of that block which is
+// row i of this (padded) front, -1 if none (a missing child has -1 throughout).
+struct Pull {
+  int64_t u[2], inv[2];
+  int32_t cld[2];
+};
+// Entry (i, j), i >= j, of a front: s plus the children's update blocks (the
+// extend-add), first child first, formed where it is used.  i0, i1 and j0, j1: its
+// row and column in the children (child_row); relpos increases, so the child's
+// entry is in its lower triangle too.
+// Without branches, so that the loads of many entries are in flight together:
+// an entry that a child does not have reads F[0] and adds zero.
+__device__ __forceinline__ double assembled(const double* F, double s, const Pull& q, int i0, int i1, int j0, int j1) {
+  const bool h0 = (i0 | j0) >= 0, h1 = (i1 | j1) >= 0;
+  const double u0 = F[h0 ? q.u[0] + i0 + (int64_t)j0 * q.cld[0] : 0];
+  const double u1 = F[h1 ? q.u[1] + i1 + (int64_t)j1 * q.cld[1] : 0];
+  s = h0 ? s + u0 : s;
+  return h1 ? s + u1 : s;
+}
+__device__ __forceinline__ int child_row(const int32_t* inv, const Pull& q, int s, int i) { return inv[q.inv[s] + i]; }
 struct Bases {
   double* p[kNumBases];
   double* ws;  // split-K partial tiles of the slot
+  const Pull* pulls;
+  const int32_t* inv;
 };
 
 // One GEMM problem: C = alpha op(A) op(B) + beta C, column-major.
@@ -42,6 +65,8 @@ struct GemmProb {
   // triangular operand, zeros skipped: 1 op(B) lower (k >= first column of
   // the tile), 2 op(A) upper (k >= first row), 3 op(A) lower (k < last row + 1)
   int8_t kmode;
+  int32_t pull;     // launches with `pull`: entry of Bases::pulls added to C
+  int32_t pull_row; // front row of C's first row and column
   double alpha, beta;
 };
 struct GemmTile {
@@ -69,6 +94,7 @@ struct GemmLaunch {
   int64_t ws_off = 0;
   // few right-hand sides (N <= kGemvMaxN, op(B) = B, general C): a
   // bandwidth-bound kernel reading A once instead of 64-wide MFMA tiles
+  bool pull = false;             // the children's update blocks are added to C (level SYRK)
   bool gemv = false;
   bool gemv_wide = false;        // narrow launch with deep K: sixteen waves share each row block's K range
 };
@@ -89,25 +115,11 @@ constexpr int kStalled = -1;  // status of a factorisation whose waits gave up
 struct FrontTask {      // i = j: the diagonal block j; else tiles (i, j), (i + 1, j)
   int32_t front, j, i, pad;
 };
-struct ExtAddDesc {     // extend-add of a child's update block into its parent
-  int64_t cfoff, pfoff, relpos_off;
-  int32_t cld, cp, pld, b;
-  int32_t split, pad;   // child columns [0, split) land in the parent's own columns
-};
-struct ExtAddTile {
-  int32_t desc, ti, tj, phase;  // phase 0: columns < split, 1: columns >= split
-};
-
 struct LevelPlan {
   std::vector<int> nodes;
-  // extend-add per child slot and phase: phase 0 (into the own columns) before
-  // the level's factorisation, phase 1 (into the update blocks) after its
-  // SYRK, which writes the update blocks without reading them
-  int next[2][2] = {{0, 0}, {0, 0}};    // [phase][slot] tile counts
-  ExtAddDesc* d_ext[2] = {nullptr, nullptr};
-  ExtAddTile* d_exttile[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-  std::vector<ExtAddDesc> h_ext[2];
-  std::vector<ExtAddTile> h_exttile[2][2];
+  // lower 64x64 tiles (node, ti, tj) of the own columns of fronts with children
+  int4* d_owntiles = nullptr;
+  int nowntiles = 0;
   // factorisation of the own columns: fronts and tasks in ticket order
   FrontDesc* d_fronts = nullptr;
   FrontTask* d_tasks = nullptr;
@@ -176,6 +188,8 @@ struct spde_plan {
   int32_t* d_relpos = nullptr;
   int32_t* d_bnd = nullptr;       // concatenated boundary lists (elimination indices)
   spde::NodeDev* d_nodes = nullptr;
+  spde::Pull* d_pulls = nullptr;  // per node
+  int32_t* d_inv = nullptr;
   double* d_tmpl = nullptr;       // per-cell value templates of the blocks of Q
   double* d_acan = nullptr;       // canonical 9-point spatial operator A
   double* d_a0can = nullptr;      // canonical 9-point initial-state operator A0

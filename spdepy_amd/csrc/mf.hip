@@ -1,5 +1,5 @@
 // Sparse <-> frontal data movement of the multifrontal method: scatter of Q
-// into the fronts, extend-add of update blocks, log-determinant reduction,
+// into the fronts, assembly of the own columns, log-determinant reduction,
 // gathers for the triangular solves and the selected inverse.
 #include <hip/hip_runtime.h>
 
@@ -23,33 +23,37 @@ __global__ void diag_add_kernel(const double* __restrict__ add, const int64_t* _
     F[map[diag[r]]] += add[r];
 }
 
-// Extend-add of the lower triangle of a child's update block (rows/cols p..n
-// of its front) into the parent front at relpos.  Tile 64x64 of the child's
-// b x b block; tiles above the diagonal are not listed.  Phase 0 adds the
-// columns that land in the parent's own columns, phase 1 the rest (into the
-// parent's update block, after the parent's SYRK has written it).
-__global__ __launch_bounds__(256) void extend_add_kernel(const ExtAddDesc* __restrict__ descs,
-                                                         const ExtAddTile* __restrict__ tiles,
-                                                         const int32_t* __restrict__ relpos,
-                                                         double* __restrict__ F) {
-  __shared__ int rpj[64];
-  const ExtAddTile t = tiles[blockIdx.x];
-  const ExtAddDesc d = descs[t.desc];
-  const int32_t* rp = relpos + d.relpos_off;
-  const double* U = F + d.cfoff + d.cp + (int64_t)d.cp * d.cld;
-  double* P = F + d.pfoff;
-  const int tid = threadIdx.x;
-  if (tid < 64) rpj[tid] = (t.tj * 64 + tid < d.b) ? rp[t.tj * 64 + tid] : -1;
+// Own columns of a level's fronts: Q's scattered values plus the children's
+// update blocks, one 64x64 tile of the lower triangle per block.  All loads of a
+// thread's sixteen entries are issued before the first store.  Both children in
+// one pass: a launch per child and phase took four dependent launches of 10 us a
+// level and read and wrote every entry of the parent twice; the update blocks are
+// assembled in the SYRK that writes them.
+__global__ __launch_bounds__(256) void own_assemble_kernel(const NodeDev* __restrict__ nodes,
+                                                           const int4* __restrict__ tiles,
+                                                           const Pull* __restrict__ pulls,
+                                                           const int32_t* __restrict__ inv, double* __restrict__ F) {
+  __shared__ int cj[2][64];
+  const int4 t = tiles[blockIdx.x];
+  const NodeDev nd = nodes[t.x];
+  const Pull q = pulls[t.x];
+  const int tid = threadIdx.x, u = tid & 63, w0 = tid >> 6;
+  const int nf = nd.pp + nd.nb, i = t.y * 64 + u;
+  if (tid < 128) cj[tid >> 6][u] = child_row(inv, q, tid >> 6, t.z * 64 + u);  // t.z * 64 + 63 < pp
+  const int i0 = i < nf ? child_row(inv, q, 0, i) : -1, i1 = i < nf ? child_row(inv, q, 1, i) : -1;
   __syncthreads();
-  const int i = t.ti * 64 + (tid & 63);
-  if (i >= d.b) return;
-  const int pi = rp[i];
-  const int jlo = t.phase ? d.split : 0, jhi = t.phase ? d.b : d.split;
-#pragma unroll 4
-  for (int jj = (tid >> 6); jj < 64; jj += 4) {
-    const int j = t.tj * 64 + jj;
-    if (j > i || j < jlo || j >= jhi) continue;
-    P[pi + (int64_t)rpj[jj] * d.pld] += U[i + (int64_t)j * d.cld];
+  double* f = F + nd.foff;
+  double v[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int c = w0 + 4 * k, j = t.z * 64 + c;
+    const bool low = j <= i && i < nf;
+    v[k] = assembled(F, low ? f[i + (int64_t)j * nd.ld] : 0.0, q, low ? i0 : -1, low ? i1 : -1, cj[0][c], cj[1][c]);
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int j = t.z * 64 + w0 + 4 * k;
+    if (j <= i && i < nf) f[i + (int64_t)j * nd.ld] = v[k];
   }
 }
 
@@ -251,9 +255,10 @@ void launch_scatter(const double* q, const int64_t* map, int64_t nnz, double* F,
 void launch_diag_add(const double* add, const int64_t* diag, const int64_t* map, int64_t n, double* F, hipStream_t s) {
   hipLaunchKernelGGL(diag_add_kernel, dim3(grid_for(n)), dim3(256), 0, s, add, diag, map, n, F);
 }
-void launch_extend_add(const ExtAddDesc* d, const ExtAddTile* t, int ntiles, const int32_t* relpos, double* F,
-                       hipStream_t s) {
-  if (ntiles > 0) hipLaunchKernelGGL(extend_add_kernel, dim3(ntiles), dim3(256), 0, s, d, t, relpos, F);
+void launch_own_assemble(const NodeDev* nodes, const int4* tiles, int ntiles, const Pull* pulls, const int32_t* inv,
+                         double* F, hipStream_t s) {
+  if (ntiles > 0)
+    hipLaunchKernelGGL(own_assemble_kernel, dim3(ntiles), dim3(256), 0, s, nodes, tiles, pulls, inv, F);
 }
 int logdet_parts(int64_t n) { return (int)((n + kLogdetPer - 1) / kLogdetPer); }
 void launch_logdet(const int64_t* diag, const int64_t* map, int64_t n, const double* F, double* partial, double* out,

@@ -14,14 +14,14 @@
 namespace spde {
 
 void launch_gemm(const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned lds = 0);
+void launch_own_assemble(const NodeDev* nodes, const int4* tiles, int ntiles, const Pull* pulls, const int32_t* inv,
+                         double* F, hipStream_t s);
 void launch_front_factor(const FrontDesc* fronts, const FrontTask* tasks, int ntasks, double* F, double* Z, int* flags,
                          int* ticket, int* stop, int* status, hipStream_t s);
 void launch_clear_flags(int* p, int n, hipStream_t s);
 void launch_fill(double* p, int64_t n, double v, hipStream_t s);
 void launch_scatter(const double* q, const int64_t* map, int64_t nnz, double* F, hipStream_t s);
 void launch_diag_add(const double* add, const int64_t* diag, const int64_t* map, int64_t n, double* F, hipStream_t s);
-void launch_extend_add(const ExtAddDesc* d, const ExtAddTile* t, int ntiles, const int32_t* relpos, double* F,
-                       hipStream_t s);
 int logdet_parts(int64_t n);
 void launch_logdet(const int64_t* diag, const int64_t* map, int64_t n, const double* F, double* partial, double* out,
                    hipStream_t s);
@@ -397,47 +397,32 @@ int build_factor_plan(spde_plan* pl) {
   for (size_t l = 0; l < sym.levels.size(); ++l) {
     LevelPlan& L = pl->levels[l];
     L.nodes = sym.levels[l];
-    for (int s = 0; s < 2; ++s) {
-      for (int id : L.nodes) {
-        const Node& nd = sym.nodes[id];
-        if (s >= nd.nchild) continue;
-        const Node& c = sym.nodes[nd.child[s]];
-        const int b = (int)c.B.size();
-        if (b == 0) continue;
-        const int di = (int)L.h_ext[s].size();
-        int split = 0;  // relpos increases: the first `split` columns map into the parent's own columns
-        while (split < b && c.relpos[split] < nd.p) ++split;
-        const FrontLay &cl = pl->lay[nd.child[s]], &fl = pl->lay[id];
-        L.h_ext[s].push_back({cl.foff, fl.foff, c.relpos_off, cl.ld, cl.pp, fl.ld, b, split, 0});
-        const int nt = (b + 63) / 64;
-        for (int a = 0; a < nt; ++a)
-          for (int bb = 0; bb <= a; ++bb) {
-            if (bb * 64 < split) L.h_exttile[0][s].push_back({di, a, bb, 0});
-            if ((bb + 1) * 64 > split) L.h_exttile[1][s].push_back({di, a, bb, 1});
-          }
-      }
-      int rc = upload(&L.d_ext[s], L.h_ext[s]);
-      if (rc) return rc;
-      for (int ph = 0; ph < 2; ++ph) {
-        L.next[ph][s] = (int)L.h_exttile[ph][s].size();
-        rc = upload(&L.d_exttile[ph][s], L.h_exttile[ph][s]);
-        if (rc) return rc;
-      }
+    std::vector<int4> own;
+    for (int id : L.nodes) {
+      const Node& nd = sym.nodes[id];
+      const FrontLay& f = pl->lay[id];
+      if (nd.nchild == 0) continue;
+      for (int ti = 0; ti * 64 < f.pp + (int)nd.B.size(); ++ti)
+        for (int tj = 0; tj <= ti && tj * 64 < f.pp; ++tj) own.push_back(make_int4(id, ti, tj, 0));
     }
-    int rcf = build_front_tasks(pl, L);
+    L.nowntiles = (int)own.size();
+    int rcf = upload(&L.d_owntiles, own);
+    if (!rcf) rcf = build_front_tasks(pl, L);
     if (rcf) return rcf;
     L.syrk.ta = false;
     L.syrk.tb = true;
+    L.syrk.pull = true;
     for (int id : L.nodes) {
       const Node& nd = sym.nodes[id];
       const FrontLay& f = pl->lay[id];
       const int n = f.ld, b = (int)nd.B.size();
-      // beta = 0: the update block is written here, the children's
-      // contributions to it are added afterwards (extend-add phase 1)
-      add_prob(L.syrk,
-               prob(kFront, f.foff + f.pp, n, kFront, f.foff + f.pp, n, kFront, f.foff + f.pp + (int64_t)f.pp * n, n,
-                    b, b, nd.p, -1.0, 0.0),
-               true);
+      // the update block is written here together with the children's
+      // contributions to it
+      GemmProb P = prob(kFront, f.foff + f.pp, n, kFront, f.foff + f.pp, n, kFront,
+                        f.foff + f.pp + (int64_t)f.pp * n, n, b, b, nd.p, -1.0, 0.0);
+      P.pull = id;
+      P.pull_row = f.pp;
+      add_prob(L.syrk, P, true);
     }
     int rc = finalize(L.syrk, &pl->split_fs);
     if (rc) return rc;
@@ -494,13 +479,6 @@ int build_factor_plan(spde_plan* pl) {
   for (auto& L : pl->levels) {
     int rc = validate(L.syrk, as, "factor syrk");
     if (rc) return rc;
-    for (int c = 0; c < 2; ++c)
-      for (const ExtAddDesc& d : L.h_ext[c])
-        if (d.cfoff + (int64_t)d.cld * (d.cp + d.b) > pl->lay_front || d.pfoff >= pl->lay_front ||
-            d.cp + d.b > d.cld) {
-          set_error("extend-add descriptor out of bounds");
-          return SPDE_ERR_STATE;
-        }
   }
   for (auto& g : pl->trtri) {
     int rc = validate(g, as, "inverse of L11");
@@ -683,6 +661,8 @@ int ensure_splitws(spde_plan* pl, int slot) {
 Bases make_bases(spde_plan* pl, int slot, double* x) {
   Bases b;
   b.ws = pl->slots[slot].splitws;
+  b.pulls = pl->d_pulls;
+  b.inv = pl->d_inv;
   b.p[kFront] = pl->slots[slot].front;
   b.p[kZ] = pl->slots[slot].z;
   b.p[kSigma] = pl->slots[slot].sigma;
@@ -831,6 +811,40 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
   TRY(upload(&pl->d_relpos, relpos));
   TRY(upload(&pl->d_bnd, bnd));
   TRY(upload(&pl->d_nodes, nodes));
+  {
+    // children's rows by row of the padded parent front
+    std::vector<Pull> pulls(sym.nodes.size());
+    int nfmax = 0;
+    for (size_t q = 0; q < sym.nodes.size(); ++q)
+      nfmax = std::max(nfmax, pl->lay[q].pp + (int)sym.nodes[q].B.size());
+    std::vector<int32_t> inv(nfmax, -1);  // the rows of a missing child
+    for (size_t q = 0; q < sym.nodes.size(); ++q) {
+      const Node& nd = sym.nodes[q];
+      Pull& P = pulls[q];
+      for (int s = 0; s < 2; ++s) {
+        P.u[s] = 0;
+        P.inv[s] = 0;
+        P.cld[s] = 0;
+        if (s >= nd.nchild || sym.nodes[nd.child[s]].B.empty()) continue;
+        const Node& c = sym.nodes[nd.child[s]];
+        const FrontLay& cl = pl->lay[nd.child[s]];
+        const int nf = pl->lay[q].pp + (int)nd.B.size();
+        P.u[s] = cl.foff + cl.pp + (int64_t)cl.pp * cl.ld;
+        P.cld[s] = cl.ld;
+        P.inv[s] = (int64_t)inv.size();
+        inv.resize(inv.size() + nf, -1);
+        for (size_t k = 0; k < c.B.size(); ++k) {
+          const int at = relpos[c.relpos_off + k];
+          if (at < 0 || at >= nf || (k && at <= relpos[c.relpos_off + k - 1]) ||
+              P.u[s] + (int64_t)(c.B.size() - 1) * (cl.ld + 1) >= pl->lay_front)
+            TRY((set_error("child rows outside the parent front"), SPDE_ERR_STATE));
+          inv[P.inv[s] + at] = (int32_t)k;
+        }
+      }
+    }
+    TRY(upload(&pl->d_pulls, pulls));
+    TRY(upload(&pl->d_inv, inv));
+  }
   TRY(upload(&ex->d_children, children));
   {
     std::vector<int4> zt;
@@ -883,7 +897,7 @@ void spde_plan_destroy(spde_plan* pl) {
     hipDeviceSynchronize();
     for (auto* p : {(void*)pl->d_indptr, (void*)pl->d_indices, (void*)pl->d_code, (void*)pl->d_diag,
                     (void*)pl->d_map, (void*)pl->d_mapsym, (void*)pl->d_perm, (void*)pl->d_relpos,
-                    (void*)pl->d_bnd, (void*)pl->d_nodes, (void*)pl->d_tmpl, (void*)pl->d_acan,
+                    (void*)pl->d_bnd, (void*)pl->d_nodes, (void*)pl->d_pulls, (void*)pl->d_inv, (void*)pl->d_tmpl, (void*)pl->d_acan,
                     (void*)pl->d_a0can, (void*)pl->d_qdiag, (void*)pl->d_win, (void*)pl->d_red, (void*)pl->d_pos25,
                     (void*)pl->d_sprow, (void*)pl->d_spcol, (void*)pl->d_gpart, (void*)pl->d_tan})
       hipFree(p);
@@ -901,13 +915,9 @@ void spde_plan_destroy(spde_plan* pl) {
       hipFree(s.splitws);
     }
     for (auto& L : pl->levels) {
-      for (int s = 0; s < 2; ++s) {
-        hipFree(L.d_ext[s]);
-        hipFree(L.d_exttile[0][s]);
-        hipFree(L.d_exttile[1][s]);
-      }
       hipFree(L.d_fronts);
       hipFree(L.d_tasks);
+      hipFree(L.d_owntiles);
       for (GemmLaunch* g : {&L.syrk, &L.si_x, &L.si_s21, &L.si_s11a, &L.si_s11b}) free_launch(*g);
     }
     for (auto& g : pl->trtri) free_launch(g);
@@ -1009,11 +1019,10 @@ int spde_factor_async(spde_plan* pl, int slot, const double* qval, const double*
   Bases b = make_bases(pl, slot, nullptr);
   for (size_t l = 0; l < pl->levels.size(); ++l) {
     LevelPlan& L = pl->levels[l];
-    for (int c = 0; c < 2; ++c) launch_extend_add(L.d_ext[c], L.d_exttile[0][c], L.next[0][c], pl->d_relpos, sl.front, s);
+    launch_own_assemble(pl->d_nodes, L.d_owntiles, L.nowntiles, pl->d_pulls, pl->d_inv, sl.front, s);
     launch_front_factor(L.d_fronts, L.d_tasks, L.ntasks, sl.front, sl.z, sl.flags + 1 + pl->levels.size(),
                         sl.flags + 1 + l, sl.flags, sl.status, s);
     run_gemm(pl, L.syrk, b, s);
-    for (int c = 0; c < 2; ++c) launch_extend_add(L.d_ext[c], L.d_exttile[1][c], L.next[1][c], pl->d_relpos, sl.front, s);
   }
   for (auto& g : pl->trtri) run_gemm(pl, g, b, s);
   launch_logdet(pl->d_diag, pl->d_map, sym.n, sl.front, sl.partial, sl.ld, s);
