@@ -15,8 +15,8 @@
 // W[16 kc + 4 (lane / 16) + j][16 h + lane % 16] (zero for k >= 9 cin), the B
 // operand of the 16x16x16 instruction for k-chunk kc and output half h.
 //
-// Each wave computes a 16-pixel x 32-channel tile: A rows are pixels (lane
-// % 16), A k-columns 4 (lane / 16) + j; D rows 4 (lane / 16) + j, columns lane % 16.
+// A wave's tiles are 16 pixels x 32 channels: A rows are pixels (lane % 16), A
+// k-columns 4 (lane / 16) + j; D rows 4 (lane / 16) + j, columns lane % 16.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -39,133 +39,212 @@ __device__ __host__ inline unsigned short to_bf16(float f) {
   return (unsigned short)(u >> 16);
 }
 
-// Convolution of one layer.  in: P x cin; mask (optional, P x cin): the input
-// is in * (mask > 0) (backward data through a ReLU); out: P x 32, out = act(D +
-// bias) with act ReLU when relu, bias optional.  nk = number of 16-wide k chunks.
-__global__ __launch_bounds__(256) void conv_kernel(int M, int N, int64_t P, int cin, int nk,
-                                                   const float* __restrict__ in, const float* __restrict__ mask,
-                                                   const unsigned short* __restrict__ frag,
-                                                   const float* __restrict__ bias, int relu, float* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t p0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
-  if (p0 >= P) return;  // whole wave
-  const int64_t MN = (int64_t)M * N;
-  const int64_t p = p0 + (lane & 15);
-  const int kq = lane >> 4;
-  const bool pv = p < P;
-  int x = 0, y = 0;
-  int64_t tb = 0;
-  if (pv) {
-    const int64_t t = p / MN, rem = p - t * MN;
-    y = (int)(rem / M);
-    x = (int)(rem - (int64_t)y * M);
-    tb = t * MN;
-  }
-  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  for (int kc = 0; kc < nk; ++kc) {
-    const int k0 = 16 * kc + 4 * kq;
-    const int tap = k0 / cin, ci = k0 - tap * cin;
-    bf16x4 a = {0, 0, 0, 0};
-    if (pv && tap < 9) {
-      const int nx = x + tap % 3 - 1, ny = y + tap / 3 - 1;
-      if (nx >= 0 && nx < M && ny >= 0 && ny < N) {
-        const int64_t q = (tb + (int64_t)ny * M + nx) * cin + ci;
+// A block works on patches of one time slice, kTx x TY pixels; the patch and its
+// one-pixel border are staged in LDS once as BF16 (masked on the way), so that
+// an activation is read from memory about 1.4 times instead of nine and converted
+// as often.  Pixel-major, the channels of a pixel contiguous, 8 bytes of padding a
+// pixel (the sixteen pixels of a fragment fall on different banks).
+constexpr int kTx = 16;
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int CIN>
+constexpr int patch_pitch = CIN + 4;  // halves per pixel
+
+// Loads rows [y0 - B, y0 + TY + B) and columns [x0 - B, x0 + kTx + B) of slice t,
+// zero outside, masked by mask > 0.  SUM: adds the thread's values to sum (its
+// channels 4 (thread % (CIN / 4)) .. + 3).
+template <int CIN, int TY, int B, int NT, bool SUM>
+__device__ __forceinline__ void load_patch(unsigned short* __restrict__ lds, const float* __restrict__ in,
+                                           const float* __restrict__ mask, int M, int N, int64_t t, int x0, int y0,
+                                           float (&sum)[4]) {
+  constexpr int W = kTx + 2 * B, H = TY + 2 * B, C4 = CIN / 4, total = W * H * C4;
+#pragma unroll 4
+  for (int c = threadIdx.x; c < total; c += NT) {
+    const int pix = c / C4, part = c - pix * C4;
+    const int py = pix / W, px = pix - py * W;
+    const int x = x0 - B + px, y = y0 - B + py;
+    f4u v = {0.f, 0.f, 0.f, 0.f};
+    if (x >= 0 && x < M && y >= 0 && y < N) {
+      const int64_t q = ((t * N + y) * (int64_t)M + x) * CIN + 4 * part;
+      v = *(const f4u*)(in + q);
+      if (mask) {
+        const f4u k = *(const f4u*)(mask + q);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float v = in[q + j];
-          if (mask && !(mask[q + j] > 0.f)) v = 0.f;
-          a[j] = (short)to_bf16(v);
-        }
+        for (int j = 0; j < 4; ++j) v[j] = k[j] > 0.f ? v[j] : 0.f;
       }
     }
+    bf16x4 h;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      h[j] = (short)to_bf16(v[j]);
+      if (SUM) sum[j] += v[j];
+    }
+    *(bf16x4*)(lds + pix * patch_pitch<CIN> + 4 * part) = h;
+  }
+}
+
+// Convolution of one layer.  in: P x CIN; mask (optional, P x CIN): the input
+// is in * (mask > 0) (backward data through a ReLU); out: P x 32, out = act(D +
+// bias) with act ReLU when relu, bias optional.  Each of the four waves takes two
+// rows of the 16 x 8 patch, 16 pixels x 32 channels per row.  HBM-bound (77 MB for
+// 200,000 pixels and 32 channels with a mask): per-lane gathers of the fragments from
+// memory took 186 us for it.
+template <int CIN>
+__global__ __launch_bounds__(256) void conv_kernel(int M, int N, int nx, int ny, const float* __restrict__ in,
+                                                   const float* __restrict__ mask,
+                                                   const unsigned short* __restrict__ frag,
+                                                   const float* __restrict__ bias, int relu, float* __restrict__ out) {
+  constexpr int TY = 8, W = kTx + 2, PP = patch_pitch<CIN>, nk = (9 * CIN + 15) / 16;
+  __shared__ __align__(16) unsigned short patch[W * (TY + 2) * PP];
+  const int64_t t = blockIdx.x / (nx * ny);
+  const int r = (int)(blockIdx.x - t * (nx * ny));
+  const int x0 = (r % nx) * kTx, y0 = (r / nx) * TY;
+  float none[4];
+  load_patch<CIN, TY, 1, 256, false>(patch, in, mask, M, N, t, x0, y0, none);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int px = lane & 15, kq = lane >> 4;
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int y = 0; y < 2; ++y)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) acc[y][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kc = 0; kc < nk; ++kc) {
+    const int k0 = 16 * kc + 4 * kq;
+    const int tap = k0 / CIN, ci = k0 - tap * CIN;
+    const int dx = tap % 3, dy = tap / 3;
     const bf16x4 b0 = *(const bf16x4*)(frag + ((int64_t)(kc * 2 + 0) * 64 + lane) * 4);
     const bf16x4 b1 = *(const bf16x4*)(frag + ((int64_t)(kc * 2 + 1) * 64 + lane) * 4);
-    acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b0, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b1, acc1, 0, 0, 0);
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      bf16x4 a = {0, 0, 0, 0};
+      if (tap < 9) a = *(const bf16x4*)(patch + ((2 * wave + y + dy) * W + px + dx) * PP + ci);
+      acc[y][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b0, acc[y][0], 0, 0, 0);
+      acc[y][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b1, acc[y][1], 0, 0, 0);
+    }
   }
   const int co = lane & 15;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t pp = p0 + 4 * kq + j;
-    if (pp >= P) continue;
-    float v0 = acc0[j] + (bias ? bias[co] : 0.f), v1 = acc1[j] + (bias ? bias[co + 16] : 0.f);
-    if (relu) {
-      v0 = v0 > 0.f ? v0 : 0.f;
-      v1 = v1 > 0.f ? v1 : 0.f;
-    }
-    out[pp * kCh + co] = v0;
-    out[pp * kCh + co + 16] = v1;
-  }
-}
-
-// Partial weight gradients over a chunk of pixels:
-// part[chunk][k][co] = sum_{p in chunk} X[p + off(tap)][ci] dZ[p][co] with
-// dZ = G (G * (Y > 0) when mask), both operands rounded to BF16 as in the
-// forward pass.  One wave per (chunk, 16 k-rows, 16 output columns).
-__global__ __launch_bounds__(64) void conv_wgrad_kernel(int M, int N, int64_t P, int cin, int64_t chunk,
-                                                        const float* __restrict__ X, const float* __restrict__ G,
-                                                        const float* __restrict__ Y, float* __restrict__ part) {
-  const int lane = threadIdx.x;
-  const int nkt = (9 * cin + 15) / 16;
-  const int tile = blockIdx.y;       // k-tile * 2 + column half
-  const int kt = tile >> 1, h = tile & 1;
-  const int64_t c0 = (int64_t)blockIdx.x * chunk;
-  const int64_t c1 = c0 + chunk < P ? c0 + chunk : P;
-  const int64_t MN = (int64_t)M * N;
-  const int krow = 16 * kt + (lane & 15);
-  const int tap = krow / cin, ci = krow - tap * cin;
-  const int co = 16 * h + (lane & 15);
-  const int kq = lane >> 4;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int64_t p0 = c0; p0 < c1; p0 += 16) {
-    bf16x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
+  for (int y = 0; y < 2; ++y) {
+    const int gy = y0 + 2 * wave + y;
+    if (gy >= N) continue;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int64_t p = p0 + 4 * kq + j;
-      if (p >= c1) continue;
-      if (tap < 9) {
-        const int64_t t = p / MN, rem = p - t * MN;
-        const int y = (int)(rem / M), x = (int)(rem - (int64_t)y * M);
-        const int nx = x + tap % 3 - 1, ny = y + tap / 3 - 1;
-        if (nx >= 0 && nx < M && ny >= 0 && ny < N) a[j] = (short)to_bf16(X[(t * MN + (int64_t)ny * M + nx) * cin + ci]);
+      const int gx = x0 + 4 * kq + j;
+      if (gx >= M) continue;
+      float v0 = acc[y][0][j] + (bias ? bias[co] : 0.f), v1 = acc[y][1][j] + (bias ? bias[co + 16] : 0.f);
+      if (relu) {
+        v0 = v0 > 0.f ? v0 : 0.f;
+        v1 = v1 > 0.f ? v1 : 0.f;
       }
-      float g = G[p * kCh + co];
-      if (Y && !(Y[p * kCh + co] > 0.f)) g = 0.f;
-      b[j] = (short)to_bf16(g);
+      float* o = out + ((t * N + gy) * (int64_t)M + gx) * kCh;
+      o[co] = v0;
+      o[co + 16] = v1;
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+  }
+}
+
+// Partial weight and bias gradients of a block's patches (patch b, b + blocks,
+// .. in order): wpart[block][k][co] = sum_p X[p + off(tap)][ci] dZ[p][co] and
+// bpart[block][co] = sum_p dZ[p][co] with dZ = G (G * (Y > 0) when Y), the operands
+// of the product rounded to BF16 as in the forward pass, the bias in FP32.  The
+// contraction runs over pixels: both fragments are gathered from the staged
+// patches, four pixels of a row to a lane; the 2 * 18 tiles of 16 x 16 weights are
+// spread over the eight waves and stay in registers.  (One wave per chunk and tile,
+// gathering from memory, took 301 us and the bias another 308.)
+template <int CIN>
+__global__ __launch_bounds__(512) void conv_wgrad_kernel(int M, int N, int nx, int ny, int npatch,
+                                                         const float* __restrict__ X, const float* __restrict__ G,
+                                                         const float* __restrict__ Y, float* __restrict__ wpart,
+                                                         float* __restrict__ bpart) {
+  constexpr int TY = 8, W = kTx + 2, PP = patch_pitch<CIN>, PG = patch_pitch<kCh>, nkt = (9 * CIN + 15) / 16;
+  constexpr int NTILE = 2 * nkt, PER = (NTILE + 7) / 8;
+  __shared__ __align__(16) unsigned short xs[W * (TY + 2) * PP];
+  __shared__ __align__(16) unsigned short gs[kTx * TY * PG];
+  __shared__ float bs[512 * 4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lr = lane & 15, kq = lane >> 4;
+  f32x4 acc[PER];
+#pragma unroll
+  for (int q = 0; q < PER; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float bsum[4] = {0.f, 0.f, 0.f, 0.f}, none[4];
+  for (int b = blockIdx.x; b < npatch; b += gridDim.x) {
+    const int64_t t = b / (nx * ny);
+    const int r = (int)(b - t * (nx * ny));
+    const int x0 = (r % nx) * kTx, y0 = (r / nx) * TY;
+    __syncthreads();
+    load_patch<CIN, TY, 1, 512, false>(xs, X, nullptr, M, N, t, x0, y0, none);
+    load_patch<kCh, TY, 0, 512, true>(gs, G, Y, M, N, t, x0, y0, bsum);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int tile = wave + 8 * q;  // k-tile * 2 + column half
+      if (tile >= NTILE) break;
+      const int krow = 16 * (tile >> 1) + lr, h = tile & 1;
+      const int tap = krow / CIN, ci = krow - tap * CIN;
+      const bool in = tap < 9;
+      const unsigned short* xp = xs + (in ? ((tap / 3) * W + tap % 3) * PP + ci : 0);
+      const unsigned short* gp = gs + 16 * h + lr;
+#pragma unroll
+      for (int y = 0; y < TY; ++y) {
+        bf16x4 a, c;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          a[j] = in ? (short)xp[(y * W + 4 * kq + j) * PP] : (short)0;
+          c[j] = (short)gp[(y * kTx + 4 * kq + j) * PG];
+        }
+        acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, c, acc[q], 0, 0, 0);
+      }
+    }
   }
   // D rows (k) 4 kq + j, column lane & 15
-  float* dst = part + (int64_t)blockIdx.x * (nkt * 16) * kCh;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) dst[(int64_t)(16 * kt + 4 * kq + j) * kCh + co] = acc[j];
-  (void)nkt;
-}
-
-// Bias gradient partials: part[chunk][co] = sum_{p in chunk} dZ[p][co].
-__global__ __launch_bounds__(64) void conv_bgrad_kernel(int64_t P, int64_t chunk, const float* __restrict__ G,
-                                                        const float* __restrict__ Y, float* __restrict__ part) {
-  const int co = threadIdx.x;
-  if (co >= kCh) return;
-  const int64_t c0 = (int64_t)blockIdx.x * chunk;
-  const int64_t c1 = c0 + chunk < P ? c0 + chunk : P;
-  float s = 0.f;
-  for (int64_t p = c0; p < c1; ++p) {
-    float g = G[p * kCh + co];
-    if (Y && !(Y[p * kCh + co] > 0.f)) g = 0.f;
-    s += g;
+  for (int q = 0; q < PER; ++q) {
+    const int tile = wave + 8 * q;
+    if (tile >= NTILE) break;
+    float* dst = wpart + ((int64_t)blockIdx.x * (nkt * 16) + 16 * (tile >> 1) + 4 * kq) * kCh + 16 * (tile & 1) + lr;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dst[j * kCh] = acc[q][j];
   }
-  part[(int64_t)blockIdx.x * kCh + co] = s;
+  // thread's channels 4 (thread % 8) .. + 3: summed over the threads in order
+#pragma unroll
+  for (int j = 0; j < 4; ++j) bs[threadIdx.x * 4 + j] = bsum[j];
+  __syncthreads();
+  if (threadIdx.x < kCh) {
+    float v = 0.f;
+    for (int q = 0; q < 64; ++q) v += bs[q * 32 + threadIdx.x];
+    bpart[(int64_t)blockIdx.x * kCh + threadIdx.x] = v;
+  }
 }
 
-// grad[e] = sum over chunks of part[c][e] in chunk order (deterministic);
-// grad may be part itself (each thread reads its column before writing it).
-__global__ void chunk_sum_kernel(int nchunk, int64_t width, const float* part, float* grad) {
-  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e >= width) return;
+// dW[e] = sum over chunks of wpart[c][e], db likewise, in a fixed order: four
+// threads take a quarter of the chunks each, 64 entries to a block.
+__global__ __launch_bounds__(256) void chunk_sum_kernel(int nchunk, int64_t width, int64_t wstride,
+                                                        const float* __restrict__ wpart,
+                                                        const float* __restrict__ bpart, float* __restrict__ dW,
+                                                        float* __restrict__ db) {
+  __shared__ float red[4][64];
+  const int l = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int64_t e = blockIdx.x * 64ll + l;
+  const int q = (nchunk + 3) / 4, c0 = g * q, c1 = min(nchunk, c0 + q);
+  const bool w = e < width, in = e < width + kCh;
+  const float* src = w ? wpart + e : bpart + (e - width);
+  const int64_t stride = w ? wstride : kCh;
   float s = 0.f;
-  for (int c = 0; c < nchunk; ++c) s += part[(int64_t)c * width + e];
-  grad[e] = s;
+  if (in) {
+#pragma unroll 8
+    for (int c = c0; c < c1; ++c) s += src[c * stride];
+  }
+  red[g][l] = s;
+  __syncthreads();
+  if (g == 0 && in) {
+    const float v = ((red[0][l] + red[1][l]) + red[2][l]) + red[3][l];
+    if (w)
+      dW[e] = v;
+    else
+      db[e - width] = v;
+  }
 }
 
 // BF16 fragments of the forward operand (transposed = 0) or of the
@@ -260,11 +339,18 @@ int spde_conv_forward(int M, int N, int T, int cin, const float* in, const float
     set_error("spde_conv_forward: invalid argument");
     return SPDE_ERR_ARG;
   }
-  const int64_t P = (int64_t)M * N * T;
-  const int nk = (9 * cin + 15) / 16;
-  const int64_t tiles = (P + 15) / 16;
-  hipLaunchKernelGGL(conv_kernel, dim3(nblk(tiles, 4)), dim3(256), 0, (hipStream_t)stream, M, N, P, cin, nk, in, mask,
-                     frag, bias, relu, out);
+  const int nx = (M + kTx - 1) / kTx, ny = (N + 7) / 8;
+  if ((int64_t)nx * ny * T > INT32_MAX) {
+    set_error("spde_conv_forward: lattice too large");
+    return SPDE_ERR_ARG;
+  }
+  const dim3 grid((unsigned)(nx * ny * T));
+  if (cin == 32)
+    hipLaunchKernelGGL(conv_kernel<32>, grid, dim3(256), 0, (hipStream_t)stream, M, N, nx, ny, in, mask, frag, bias,
+                       relu, out);
+  else
+    hipLaunchKernelGGL(conv_kernel<8>, grid, dim3(256), 0, (hipStream_t)stream, M, N, nx, ny, in, mask, frag, bias,
+                       relu, out);
   SPDE_HIP(hipGetLastError());
   return SPDE_OK;
 }
@@ -289,19 +375,24 @@ int spde_conv_backward(int M, int N, int T, int cin, const float* X, const float
   hipStream_t s = (hipStream_t)stream;
   const int64_t P = (int64_t)M * N * T;
   const int64_t nchunk = P / 1024 + 1 < 256 ? P / 1024 + 1 : 256;
-  int64_t chunk = (P + nchunk - 1) / nchunk;
-  chunk = (chunk + 15) / 16 * 16;
   const int nkt = (9 * cin + 15) / 16;
   float* wpart = work;
   float* bpart = work + nchunk * (int64_t)nkt * 16 * kCh;
-  hipLaunchKernelGGL(conv_wgrad_kernel, dim3((unsigned)nchunk, (unsigned)(2 * nkt)), dim3(64), 0, s, M, N, P, cin,
-                     chunk, X, G, Y, wpart);
-  hipLaunchKernelGGL(conv_bgrad_kernel, dim3((unsigned)nchunk), dim3(64), 0, s, P, chunk, G, Y, bpart);
+  const int nx = (M + kTx - 1) / kTx, ny = (N + 7) / 8;
+  if ((int64_t)nx * ny * T > INT32_MAX) {
+    set_error("spde_conv_backward: lattice too large");
+    return SPDE_ERR_ARG;
+  }
+  if (cin == 32)
+    hipLaunchKernelGGL(conv_wgrad_kernel<32>, dim3((unsigned)nchunk), dim3(512), 0, s, M, N, nx, ny, nx * ny * T, X, G,
+                       Y, wpart, bpart);
+  else
+    hipLaunchKernelGGL(conv_wgrad_kernel<8>, dim3((unsigned)nchunk), dim3(512), 0, s, M, N, nx, ny, nx * ny * T, X, G,
+                       Y, wpart, bpart);
   // only k < 9 cin rows are real weights
-  hipLaunchKernelGGL(chunk_sum_kernel, dim3(nblk((int64_t)nkt * 16 * kCh, 256)), dim3(256), 0, s, (int)nchunk,
-                     (int64_t)nkt * 16 * kCh, wpart, wpart);
-  SPDE_HIP(hipMemcpyAsync(dW, wpart, sizeof(float) * 9 * cin * kCh, hipMemcpyDeviceToDevice, s));
-  hipLaunchKernelGGL(chunk_sum_kernel, dim3(1), dim3(64), 0, s, (int)nchunk, (int64_t)kCh, bpart, db);
+  const int64_t width = 9ll * cin * kCh;
+  hipLaunchKernelGGL(chunk_sum_kernel, dim3(nblk(width + kCh, 64)), dim3(256), 0, s, (int)nchunk, width,
+                     (int64_t)nkt * 16 * kCh, wpart, bpart, dW, db);
   SPDE_HIP(hipGetLastError());
   return SPDE_OK;
 }
