@@ -197,9 +197,22 @@ class Engine:
         if closed:
             # Critical path: factorisation of Q_c on this stream, then its
             # selected inverse on the side stream (waiting on an event
-            # recorded just before).  The solve for mu_c and the one-slice
-            # log|Q| work follow here, concurrent with the selected inverse.
+            # recorded just before).  The one-slice log|Q| work needs only the
+            # assembly: it runs on the side stream beside the factorisation.
+            # The solve for mu_c follows here, concurrent with the selected
+            # inverse.
+            assembled = torch.cuda.Event()
+            assembled.record(main)
+            side.wait_event(assembled)
             self.plan.factor_async(1, qval, diag_add)
+            with torch.cuda.stream(side):
+                q0 = sp.assemble_spatial(self.plan, 0)
+                gram = sp.assemble_spatial(self.plan, 1)
+                sp.factor_async(0, q0, owner=self)
+                sp.factor_async(1, gram, owner=self)
+                if sel:
+                    sp.selinv(0, s_q0)
+                    sp.selinv(1, s_gram)
             if sel:
                 factored = torch.cuda.Event()
                 factored.record(main)
@@ -208,13 +221,6 @@ class Engine:
                     self.plan.selinv(1, sqc)
             mu = self.plan.solve(1, b_dev)
             qmu = self.plan.spmv(qval, mu)
-            q0 = sp.assemble_spatial(self.plan, 0)
-            gram = sp.assemble_spatial(self.plan, 1)
-            sp.factor_async(0, q0, owner=self)
-            sp.factor_async(1, gram, owner=self)
-            if sel:
-                sp.selinv(0, s_q0)
-                sp.selinv(1, s_gram)
         else:
             # the reference's route: Q factorised (and inverted) on the side stream
             ready = torch.cuda.Event()
