@@ -50,6 +50,14 @@ struct IcShared {
   const double* qval = nullptr;      // Q values of the last factorisation (structural order)
   const double* diag_add = nullptr;
   bool factored = false;
+  int strip_ny = 0;                  // lines per strip of the one-column sweeps (0: colour by colour)
+  int strip_slots = 0;               // in-slice entries of a slice per direction in the strips' layout
+  int16_t* d_edelta[2] = {nullptr, nullptr};  // column - row of each, and its value
+  float* d_evalue[2] = {nullptr, nullptr};
+  void* d_slists = nullptr;          // StripList: kind (even forward, odd, even backward) x strip x direction
+  uint16_t* d_scell = nullptr;
+  int32_t* d_srow = nullptr;
+  int32_t* d_esrc[2] = {nullptr, nullptr};    // entry of l32 / u32, -1: none
 };
 // Host copies of the lists (spde_ic_export), kept by the handle that built them.
 struct IcHost {
@@ -407,6 +415,198 @@ __global__ __launch_bounds__(256) void bwd1_kernel(int64_t r0, int64_t r1, const
   float acc = strided_dot(uptr[i] + lane, uptr[i + 1], ucol, u32, x);
   for (int o = kRowLanes / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kRowLanes);
   if (lane == 0) x[i] = (y[i] - acc) * dinv[i];
+}
+// The preconditioner for one right-hand side in five launches instead of one
+// per colour (35 dependent launches of 4.2 us, 150 of the 200 us of an
+// iteration at 100x100x20, each moving under 2 MB).  Even slices hold the
+// colours 0..8, odd ones 9..17, so a slice's rows couple to the other parity only
+// across the colour halves:
+//   forward on the even slices -> r_odd -= L_oe y -> forward and backward on the
+//   odd slices -> y_even -= L_oe^T x -> backward on the even slices.
+// Inside a slice a chain of decreasing (increasing) colours changes its line only
+// when j mod 3 changes, twice at most and by two lines each, so the rows of a
+// strip of lines follow from the four lines beside it (eight for forward and
+// backward): a block takes a strip with that border, keeps it in LDS and runs all
+// nine colours behind its own barriers, recomputing those lines of the border that
+// the owned ones follow from.  A column outside the block's lines is met only in
+// rows that nothing owned follows from, and is left out.
+// The in-slice entries are kept a second time in the order a block reads them
+// (slot by slot over the rows of a slice and colour, a row's unused slots zero), so
+// that a lane has a row, its loads are coalesced and take one address each, and
+// nothing is tested.  At 100x100x20 (250 blocks of four lines) the three launches
+// take 17, 31 and 17 us and the two couplings 8.5 us each, 82 us for 150 us of
+// colour launches; what bounds them is a colour's chain of LDS reads and sums, about
+// 1.5 us, with three waves of rows to a block.  Reading the rows' own lists with
+// two, four or eight lanes a row took 25 + 56 + 26, 18 + 43 + 20 and 29 us on
+// average, two lanes a row in this layout 18 + 34 + 18.
+constexpr int kStripThreads = 256;
+constexpr int kStripHalo = 4;
+constexpr int kStripSlots = 24;  // longest in-slice list
+constexpr size_t kStripLds = 64 * 1024;
+// Neighbours of cell (i, j) in one adjacent slice (3 x 3 window, no wrap).
+__device__ __host__ inline int cross_count(int i, int j, int M, int N) {
+  return (3 - (i == 0) - (i == M - 1)) * (3 - (j == 0) - (j == N - 1));
+}
+// Slots of in-slice colour k: forward five columns on each line of a lower class
+// within two lines and those of a lower class on the own line; backward the rest.
+__device__ __host__ inline int strip_slots(int k, int dir) {
+  const int lo = 10 * (k / 3) + 2 * (k % 3);
+  return dir == 0 ? lo : kStripSlots - lo;
+}
+__device__ __host__ inline int class_size(int n, int c) { return c < n ? (n - 1 - c) / 3 + 1 : 0; }
+// Cells of a block by colour (off[k] .. off[k + 1] from `start`) that one sweep of
+// its strip computes: the owned lines and those they follow from.  The same for every
+// slice of a parity, so they are listed once on the host (worked out in the
+// kernel they took half of its time).
+struct StripList {
+  int32_t off[10], start;
+};
+struct StripArgs {
+  int M, N, T, ny, parity, halo, fwd, bwd, slots;
+  const int16_t* delta[2];
+  const float* value[2];
+  const float* dinv;
+  const StripList* lists;  // of this launch's kind, two per strip
+  const uint16_t* cell;
+  const int32_t* row;
+};
+__global__ void strip_values_kernel(int64_t n, const int32_t* __restrict__ src, const float* __restrict__ from,
+                                    float* __restrict__ to) {
+  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (e < n) to[e] = src[e] >= 0 ? from[src[e]] : 0.f;
+}
+__global__ __launch_bounds__(kStripThreads) void strip1_kernel(StripArgs A, const float* __restrict__ in,
+                                                               float* __restrict__ out) {
+  extern __shared__ float strip_lds[];
+  const int M = A.M, N = A.N, nstrip = (N + A.ny - 1) / A.ny;
+  const int t = 2 * (int)(blockIdx.x / nstrip) + A.parity, ys = (int)(blockIdx.x % nstrip) * A.ny;
+  const int ye = min(N, ys + A.ny), ylo = max(0, ys - A.halo), yhi = min(N, ye + A.halo);
+  const int cnt = (yhi - ylo) * M;
+  const int64_t base = ((int64_t)t * N + ylo) * M;
+  // a cell's value, 1 / L_ii, and by colour the cells and their rows in the slot
+  // order (v between two guards of zeros: a column outside the block's lines, met
+  // only in rows that nothing owned follows from, reads one of them)
+  const int guard = 2 * M + 2;
+  float* v = strip_lds + guard;
+  float* d = v + cnt + guard;
+  int* erow = (int*)(d + cnt);
+  unsigned short* ord = (unsigned short*)(erow + cnt);
+  const int tid = threadIdx.x;
+  for (int e = tid; e < guard; e += kStripThreads) v[e - guard] = v[cnt + e] = 0.f;
+  for (int e = tid; e < cnt; e += kStripThreads) {
+    v[e] = in[base + e];
+    d[e] = A.dinv[base + e];
+  }
+  for (int dir = 0; dir < 2; ++dir) {
+    if (!(dir == 0 ? A.fwd : A.bwd)) continue;
+    const StripList& list = A.lists[2 * (blockIdx.x % nstrip) + dir];
+    const int* off = list.off;
+    for (int e = tid; e < off[9]; e += kStripThreads) {
+      ord[e] = A.cell[list.start + e];
+      erow[e] = A.row[list.start + e];
+    }
+    __syncthreads();
+    const char* dp = (const char*)(A.delta[dir] + (int64_t)t * A.slots);
+    const char* vp = (const char*)(A.value[dir] + (int64_t)t * A.slots);
+    struct Unit {
+      int l, delta[kStripSlots];
+      float w[kStripSlots];
+    };
+    // entries of row position r of colour k, whose slots begin at s0
+    auto fetch = [&](int k, int r, int s0, Unit& u) {
+      const int rows = class_size(N, k / 3) * class_size(M, k % 3), n = strip_slots(k, dir);
+      const bool in_list = r < off[k + 1];
+      u.l = in_list ? ord[r] : -1;
+      const uint32_t at = in_list ? (uint32_t)erow[r] : 0u;
+#pragma unroll
+      for (int q = 0; q < kStripSlots; q += 2) {
+        if (q < n) {
+          const int64_t e0 = s0 + (int64_t)q * rows, e1 = e0 + rows;  // uniform
+          u.delta[q] = *(const int16_t*)(dp + 2 * e0 + 2u * at);
+          u.w[q] = *(const float*)(vp + 4 * e0 + 4u * at);
+          u.delta[q + 1] = *(const int16_t*)(dp + 2 * e1 + 2u * at);
+          u.w[q + 1] = *(const float*)(vp + 4 * e1 + 4u * at);
+        }
+      }
+    };
+    auto sweep = [&](int k, const Unit& u) {
+      const int n = strip_slots(k, dir), l = max(u.l, 0);
+      float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+      for (int q = 0; q < kStripSlots; q += 2) {
+        if (q < n) {
+          a0 += u.w[q] * v[l + u.delta[q]];
+          a1 += u.w[q + 1] * v[l + u.delta[q + 1]];
+        }
+      }
+      if (u.l >= 0) v[l] = (v[l] - (a0 + a1)) * d[l];
+    };
+    // units of a block's threads, colour after colour; the next unit's entries are
+    // loaded before this one's use (they do not depend on the sweep)
+    auto live = [](int k) { return k >= 0 && k < 9; };
+    auto width = [&](int k) { return strip_slots(k, dir) * class_size(N, k / 3) * class_size(M, k % 3); };
+    auto advance = [&](int& k, int& r0, int& s0) {
+      r0 += kStripThreads;
+      while (live(k) && r0 >= off[k + 1]) {
+        if (dir == 0) {
+          s0 += width(k);
+          ++k;
+        } else if (--k >= 0) {
+          s0 -= width(k);
+        }
+        r0 = live(k) ? off[k] : 0;
+      }
+    };
+    int k = dir == 0 ? 0 : 8, r0 = off[k] - kStripThreads, s0 = dir == 0 ? 0 : A.slots - width(8);
+    advance(k, r0, s0);
+    Unit ua, ub;
+    auto one = [&](const Unit& cur, Unit& next) {
+      const int now = k;
+      advance(k, r0, s0);
+      if (live(k)) fetch(k, r0 + tid, s0, next);
+      sweep(now, cur);
+      if (k != now) __syncthreads();
+    };
+    if (live(k)) fetch(k, r0 + tid, s0, ua);
+    while (live(k)) {
+      one(ua, ub);
+      if (live(k)) one(ub, ua);
+    }
+    __syncthreads();
+  }
+  for (int e = (ys - ylo) * M + tid; e < (ye - ylo) * M; e += kStripThreads) out[base + e] = v[e];
+}
+// The coupling of the two halves, kRowLanes lanes per row of one parity
+// (blockIdx.y: its slices):
+// parity 1: tmp_i = r_i - sum over the adjacent slices' L_ij tmp_j;
+// parity 0: tmp_i -= sum over the adjacent slices' L_ji x_j.
+__global__ __launch_bounds__(256) void cross1_kernel(int M, int N, int T, int parity, const int64_t* __restrict__ ptr,
+                                                     const int32_t* __restrict__ col, const float* __restrict__ val,
+                                                     const float* r, const float* x, float* tmp) {
+  const unsigned rem = (blockIdx.x * 256 + threadIdx.x) / kRowLanes;
+  const int lane = (int)(threadIdx.x % kRowLanes), t = 2 * (int)blockIdx.y + parity;
+  if (rem >= (unsigned)(M * N)) return;  // uniform over the group
+  const int i = t * M * N + (int)rem;
+  const int j = rem / (unsigned)M, cc = cross_count((int)rem - j * M, j, M, N);
+  const int before = t > 0 ? cc : 0, after = t + 1 < T ? cc : 0;
+  // lower lists of odd rows: both slices in front; upper lists of even rows: in
+  // front and at the end
+  const int b0 = (int)ptr[i], b1 = parity ? b0 + before : (int)ptr[i + 1] - after;
+  int p[3];
+  float w[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const int e = lane + q * kRowLanes;
+    p[q] = e < before ? b0 + e : (e < before + after ? b1 + (e - before) : -1);
+    const int at = max(p[q], 0);
+    w[q] = p[q] < 0 ? 0.f : val[at];
+    p[q] = p[q] < 0 ? -1 : col[at];
+  }
+  float acc = 0.f;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) acc += p[q] < 0 ? 0.f : w[q] * x[max(p[q], 0)];
+  for (int o = kRowLanes / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kRowLanes);
+  if (lane == 0) tmp[i] = r[i] - acc;
 }
 // y = A x for one right-hand side, a group of kRowLanes lanes per row (grid-
 // stride over the rows); the block partials of x^T y as spmm32_kernel's.
@@ -1130,9 +1330,180 @@ int ic_bwd(spde_ic* ic, const float* y, float* x, int logk, hipStream_t s, bool 
   }
   return SPDE_OK;
 }
+// LDS of a strip block with `lines` lines: 16 bytes a cell and the guards.
+size_t strip_bytes(int M, int lines) { return 16 * (size_t)M * lines + 2 * sizeof(float) * (2 * (size_t)M + 2); }
+// One right-hand side through strips of lines (strip1_kernel); tmp: n floats that
+// are neither r nor z.
+void ic_apply_strips(spde_ic* ic, const float* r, float* z, float* tmp, hipStream_t s) {
+  const int M = ic->M, N = ic->N, T = ic->T, ny = ic->strip_ny, nstrip = (N + ny - 1) / ny;
+  const int even = (T + 1) / 2, odd = T / 2;
+  const int64_t Ns = (int64_t)M * N;
+  StripArgs A{M, N, T, ny, 0, kStripHalo, 1, 0, ic->strip_slots, {ic->d_edelta[0], ic->d_edelta[1]},
+              {ic->d_evalue[0], ic->d_evalue[1]}, ic->d_dinv, (const StripList*)ic->d_slists, ic->d_scell, ic->d_srow};
+  auto lds = [&](int halo) { return strip_bytes(M, std::min(N, ny + 2 * halo)); };
+  hipLaunchKernelGGL(strip1_kernel, dim3(nstrip * even), dim3(kStripThreads), lds(A.halo), s, A, r, tmp);
+  if (odd > 0) {
+    hipLaunchKernelGGL(cross1_kernel, dim3(blocks_of(Ns * kRowLanes), odd), dim3(256), 0, s, M, N, T, 1, ic->d_lptr,
+                       ic->d_lcol, ic->d_l32, r, tmp, tmp);
+    StripArgs B = A;
+    B.parity = 1;
+    B.halo = 2 * kStripHalo;
+    B.bwd = 1;
+    B.lists += 2 * nstrip;
+    hipLaunchKernelGGL(strip1_kernel, dim3(nstrip * odd), dim3(kStripThreads), lds(B.halo), s, B, tmp, z);
+    hipLaunchKernelGGL(cross1_kernel, dim3(blocks_of(Ns * kRowLanes), even), dim3(256), 0, s, M, N, T, 0, ic->d_uptr,
+                       ic->d_ucol, ic->d_u32, tmp, z, tmp);
+  }
+  A.fwd = 0;
+  A.bwd = 1;
+  A.lists += 4 * nstrip;
+  hipLaunchKernelGGL(strip1_kernel, dim3(nstrip * even), dim3(kStripThreads), lds(A.halo), s, A, tmp, z);
+}
+// Lines per strip: about one block per CU over the slices of a parity, at most
+// what 64 KB of LDS hold with the wider border; 0 where three lines do not fit, on
+// periodic lattices, and where the lists are not laid out as the strips read
+// them (checked for every row).
+int strip_lines(const spde_ic* ic) {
+  const int M = ic->M, N = ic->N, T = ic->T;
+  if (ic->pl->lat.bc == 2 || M < 2 || N < 2 || ic->nlow >= (1 << 30) || T > 65535) return 0;
+  const int64_t Ns = (int64_t)M * N;
+  if ((int64_t)M * 4 * kStripHalo > 4096 || Ns * kStripSlots > INT32_MAX) return 0;  // does not fit, 16-bit cells
+  for (int64_t v = 0; v < ic->n; ++v) {
+    const int t = (int)(v / Ns), rem = (int)(v % Ns), x = cross_count(rem % M, rem / M, M, N);
+    const int before = t > 0 ? x : 0, after = t + 1 < T ? x : 0;
+    const int64_t l0 = ic->h_lptr[v], l1 = ic->h_lptr[v + 1], u0 = ic->h_uptr[v], u1 = ic->h_uptr[v + 1];
+    const int64_t lf = t % 2 ? before + after : 0, uf = t % 2 ? 0 : before, ub = t % 2 ? 0 : after;
+    if (l1 - l0 < lf || u1 - u0 < uf + ub || l1 - l0 - lf > 24 || u1 - u0 - uf - ub > 24) return 0;
+    const int64_t first = t * Ns;
+    auto here = [&](int64_t c) { return c >= first && c < first + Ns; };
+    for (int64_t p = l0; p < l1; ++p)
+      if (here(ic->h_lcol[p]) != (p >= l0 + lf)) return 0;
+    for (int64_t p = u0; p < u1; ++p)
+      if (here(ic->h_ucol[p]) != (p >= u0 + uf && p < u1 - ub)) return 0;
+  }
+  int fit = 0;  // longest strip whose block with the wider border (or the whole slice) fits
+  while (fit < N && strip_bytes(M, std::min(N, fit + 1 + 4 * kStripHalo)) <= kStripLds) ++fit;
+  const int want = (int)(((int64_t)N * ((T + 1) / 2) + 255) / 256);
+  const int ny = std::min(std::max(want, 3), fit);
+  return ny >= 3 || ny == N ? ny : 0;
+}
+// The strips' layout of the in-slice entries (checked: every entry has a slot).
+int build_strips(spde_ic* ic) {
+  ic->strip_ny = strip_lines(ic);
+  if (!ic->strip_ny) return SPDE_OK;
+  const int M = ic->M, N = ic->N, T = ic->T;
+  const int64_t Ns = (int64_t)M * N;
+  int64_t at[2][10];
+  for (int dir = 0; dir < 2; ++dir) {
+    at[dir][0] = 0;
+    for (int k = 0; k < 9; ++k)
+      at[dir][k + 1] = at[dir][k] + (int64_t)strip_slots(k, dir) * class_size(N, k / 3) * class_size(M, k % 3);
+  }
+  // the longer of the two directions' slices, for both
+  const int64_t slots = std::max(at[0][9], at[1][9]);
+  if (slots * T > INT32_MAX) {
+    ic->strip_ny = 0;
+    return SPDE_OK;
+  }
+  for (int dir = 0; dir < 2; ++dir) {
+    std::vector<int16_t> delta(slots * T, 0);
+    std::vector<int32_t> src(slots * T, -1);
+    const auto& ptr = dir == 0 ? ic->h_lptr : ic->h_uptr;
+    const auto& col = dir == 0 ? ic->h_lcol : ic->h_ucol;
+    for (int64_t v = 0; v < ic->n; ++v) {
+      const int64_t t = v / Ns;
+      const int rem = (int)(v % Ns), i = rem % M, j = rem / M, k = i % 3 + 3 * (j % 3);
+      const int64_t rows = (int64_t)class_size(N, k / 3) * class_size(M, k % 3);
+      const int64_t row = (int64_t)(j / 3) * class_size(M, k % 3) + i / 3;
+      int q = 0;
+      for (int64_t p = ptr[v]; p < ptr[v + 1]; ++p) {
+        if (col[p] < t * Ns || col[p] >= (t + 1) * Ns) continue;
+        if (q >= strip_slots(k, dir)) {  // not the 5 x 5 pattern: colour by colour
+          ic->strip_ny = 0;
+          return SPDE_OK;
+        }
+        // the backward direction's slices end at `slots` (they are walked from the end)
+        const int64_t s = t * slots + (dir == 0 ? 0 : slots - at[1][9]) + at[dir][k] + q * rows + row;
+        delta[s] = (int16_t)(col[p] - v);
+        src[s] = (int32_t)p;
+        ++q;
+      }
+    }
+    int rc = upload_vec(&ic->d_edelta[dir], delta);
+    if (!rc) rc = upload_vec(&ic->d_esrc[dir], src);
+    if (rc) return rc;
+    SPDE_HIP(hipMalloc((void**)&ic->d_evalue[dir], sizeof(float) * std::max<int64_t>(slots * T, 1)));
+  }
+  ic->strip_slots = (int)slots;
+  // cells of each strip: forward (decreasing class j mod 3) a line of class 1 or 0
+  // beside a needed line of a higher class, backward a line of a higher class
+  // beside a needed one of a lower; forward and backward in one launch, the
+  // forward lines of all backward ones.  Lines further than two apart do not couple.
+  const int ny = ic->strip_ny, nstrip = (N + ny - 1) / ny;
+  std::vector<StripList> lists;
+  std::vector<uint16_t> cell;
+  std::vector<int32_t> row;
+  for (int kind = 0; kind < 3; ++kind)
+    for (int st = 0; st < nstrip; ++st) {
+      const int halo = kind == 1 ? 2 * kStripHalo : kStripHalo;
+      const int ys = st * ny, ye = std::min(N, ys + ny), ylo = std::max(0, ys - halo), yhi = std::min(N, ye + halo);
+      std::vector<char> use[2];
+      for (auto& u : use) u.assign(N, 0);
+      auto close = [&](std::vector<char>& u, int from, int step) {  // classes from, from + step, from + 2 step
+        for (int c = from + step; c >= 0 && c < 3; c += step)
+          for (int j = 0; j < N; ++j) {
+            if (j % 3 != c) continue;
+            for (int m = std::max(0, j - 2); m <= std::min(N - 1, j + 2); ++m)
+              if (u[m] && (m % 3 - c) * step < 0) u[j] = 1;
+          }
+      };
+      for (int j = ys; j < ye; ++j) use[1][j] = 1;
+      if (kind > 0) close(use[1], 0, 1);
+      use[0] = use[1];
+      close(use[0], 2, -1);
+      for (int dir = 0; dir < 2; ++dir) {
+        StripList L{};
+        L.start = (int32_t)cell.size();
+        for (int k = 0; k < 9; ++k) {
+          L.off[k] = (int32_t)cell.size() - L.start;
+          if ((kind == 0 && dir == 1) || (kind == 2 && dir == 0)) continue;  // not swept
+          for (int j = 0; j < N; ++j) {
+            if (!use[dir][j] || j % 3 != k / 3) continue;
+            if (j < ylo || j >= yhi) {  // the border is too narrow: colour by colour
+              ic->strip_ny = 0;
+              return SPDE_OK;
+            }
+            for (int i = k % 3; i < M; i += 3) {
+              cell.push_back((uint16_t)((j - ylo) * M + i));
+              row.push_back((int32_t)(j / 3 * class_size(M, k % 3) + i / 3));
+            }
+          }
+        }
+        L.off[9] = (int32_t)cell.size() - L.start;
+        lists.push_back(L);
+      }
+    }
+  int rc = upload_vec((StripList**)&ic->d_slists, lists);
+  if (!rc) rc = upload_vec(&ic->d_scell, cell);
+  if (!rc) rc = upload_vec(&ic->d_srow, row);
+  return rc;
+}
+// The factor's values in that layout, after its FP32 copies are made.
+void fill_strips(spde_ic* ic, hipStream_t s) {
+  if (!ic->strip_ny) return;
+  const int64_t n = (int64_t)ic->strip_slots * ic->T;
+  for (int dir = 0; dir < 2; ++dir)
+    hipLaunchKernelGGL(strip_values_kernel, dim3(blocks_of(n)), dim3(256), 0, s, n, ic->d_esrc[dir],
+                       dir == 0 ? ic->d_l32 : ic->d_u32, ic->d_evalue[dir]);
+}
 // z = M^-1 r = (L L^T)^-1 r: forward from r into z, then backward in place,
-// the last colour's two steps in one launch.
-int ic_apply(spde_ic* ic, const float* r, float* z, int logk, hipStream_t s, unsigned lds = 0) {
+// the last colour's two steps in one launch; one right-hand side in strips when
+// the caller has a vector to spare.
+int ic_apply(spde_ic* ic, const float* r, float* z, int logk, hipStream_t s, unsigned lds = 0, float* tmp = nullptr) {
+  if (logk == 0 && tmp && ic->strip_ny > 0) {
+    ic_apply_strips(ic, r, z, tmp, s);
+    return SPDE_OK;
+  }
   ic_fwd(ic, r, z, logk, s, true, lds);
   return ic_bwd(ic, z, z, logk, s, true, lds);
 }
@@ -1178,7 +1549,10 @@ void free_shared(spde_ic* ic) {
   for (void* p : {(void*)ic->d_crow, (void*)ic->d_lptr, (void*)ic->d_uptr, (void*)ic->d_lsrc, (void*)ic->d_ulow,
                   (void*)ic->d_lch, (void*)ic->d_lcol, (void*)ic->d_lkey, (void*)ic->d_ucol, (void*)ic->d_l64,
                   (void*)ic->d_dg64,
-                  (void*)ic->d_adiag, (void*)ic->d_l32, (void*)ic->d_u32, (void*)ic->d_dinv, (void*)ic->d_qc32})
+                  (void*)ic->d_adiag, (void*)ic->d_l32, (void*)ic->d_u32, (void*)ic->d_dinv, (void*)ic->d_qc32,
+                  (void*)ic->d_edelta[0], (void*)ic->d_edelta[1], (void*)ic->d_evalue[0], (void*)ic->d_evalue[1],
+                  (void*)ic->d_esrc[0], (void*)ic->d_esrc[1], ic->d_slists, (void*)ic->d_scell,
+                  (void*)ic->d_srow})
     if (p) hipFree(p);
 }
 // A view takes its parent's pattern and factor at the start of every call.
@@ -1218,7 +1592,7 @@ void enqueue_iteration(spde_ic* ic, int logk, unsigned g, float* X, hipStream_t 
   launch_spmm(ic, logk, g, P, Qv, ic->d_part, s, lds);
   hipLaunchKernelGGL(pcg_alpha_kernel, dim3(k), dim3(kRedThreads), 0, s, (int)g, ic->d_part, ic->d_scal, ic->d_active);
   hipLaunchKernelGGL(pcg_update_kernel, dim3(g), dim3(256), lds, s, units, logk, ic->d_scal, P, Qv, X, R);
-  ic_apply(ic, R, Z, logk, s, lds);
+  ic_apply(ic, R, Z, logk, s, lds, Qv);
   hipLaunchKernelGGL(dot2_kernel, dim3(g), dim3(256), lds, s, units, logk, R, Z, ic->d_part);
   hipLaunchKernelGGL(pcg_beta_kernel, dim3(k), dim3(kRedThreads), 0, s, (int)g, ic->d_part, ic->d_scal, ic->d_active,
                      ic->d_iters, hist, cap);
@@ -1266,7 +1640,7 @@ int pcg_run(spde_ic* ic, const float* B, float* X, int logk, double tol, int max
   const unsigned g = grid_for(units);
   hipLaunchKernelGGL(fill_kernel, dim3(g), dim3(256), 0, s, units, 0.f, X);
   hipLaunchKernelGGL(copy_kernel, dim3(g), dim3(256), 0, s, units, B, R);
-  ic_apply(ic, R, Z, logk, s);
+  ic_apply(ic, R, Z, logk, s, 0, P + n * 64);
   hipLaunchKernelGGL(dot2_kernel, dim3(g), dim3(256), 0, s, units, logk, R, Z, ic->d_part);
   hipLaunchKernelGGL(pcg_init_scalars_kernel, dim3(k), dim3(kRedThreads), 0, s, (int)g, ic->d_part, tol * tol, ic->d_scal,
                      ic->d_active, ic->d_iters);
@@ -1445,6 +1819,7 @@ int spde_ic_create(spde_plan* pl, spde_ic** out) {
     spde_ic_destroy(ic);
     return code;
   };
+  if ((rc = build_strips(ic))) return fail(rc);
   if ((rc = upload_vec(&ic->d_crow, crow))) return fail(rc);
   if ((rc = upload_vec(&ic->d_lptr, ic->h_lptr))) return fail(rc);
   if ((rc = upload_vec(&ic->d_uptr, ic->h_uptr))) return fail(rc);
@@ -1603,6 +1978,7 @@ int spde_ic_correct(spde_ic* ic, const float* corr, double* logdet_m, void* stre
   hipLaunchKernelGGL(ic_cast_upper_kernel, dim3(blocks_of(ic->nlow)), dim3(256), 0, s, ic->nlow, ic->d_ulow,
                      ic->d_l64, ic->d_u32);
   hipLaunchKernelGGL(ic_cast_diag_kernel, dim3(blocks_of(n)), dim3(256), 0, s, n, ic->d_dg64, ic->d_dinv);
+  fill_strips(ic, s);
   const unsigned g = grid_for(n);
   hipLaunchKernelGGL(logdet_diag_kernel, dim3(g), dim3(256), 0, s, n, ic->d_dg64, ic->d_part);
   hipLaunchKernelGGL(sum_one_kernel, dim3(1), dim3(kRedThreads), 0, s, (int)g, ic->d_part, ic->d_scal + S_X * 64);
@@ -1795,7 +2171,7 @@ int spde_pcg_replace(spde_ic* ic, const double* b, double* x, double tol, double
   // r32 = r64, z = M^-1 r32 and the partials of r^T z, r^T r
   auto precondition = [&]() {
     hipLaunchKernelGGL(cast_down_kernel, dim3(g), dim3(256), 0, s, n, ic->d_r64, R);
-    ic_apply(ic, R, Z, 0, s);
+    ic_apply(ic, R, Z, 0, s, 0, P + n * 64);
     hipLaunchKernelGGL(dot2_kernel, dim3(g), dim3(256), 0, s, n, 0, R, Z, ic->d_part);
   };
   // a fresh recurrence from the current residual (tolerance 0: the host ends the solve)
@@ -1907,7 +2283,7 @@ int spde_pcg_replace_block(spde_ic* ic, const double* B, double* X, int k, doubl
   // r32 = r64, z = M^-1 r32, partials of r^T z and r^T r
   auto precondition = [&]() {
     hipLaunchKernelGGL(cast_down_kernel, dim3(g), dim3(256), 0, s, units, ic->d_r64, R);
-    ic_apply(ic, R, Z, logk, s);
+    ic_apply(ic, R, Z, logk, s, 0, P + n * 64);
     hipLaunchKernelGGL(dot2_kernel, dim3(g), dim3(256), 0, s, units, logk, R, Z, ic->d_part);
   };
   hipLaunchKernelGGL(fill64_kernel, dim3(g), dim3(256), 0, s, units, X);

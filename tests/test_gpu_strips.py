@@ -1,0 +1,35 @@
+"""The one-column preconditioner in strips of lines against the colour-by-colour
+sweeps that two equal columns take: the same few PCG iterations."""
+import numpy as np
+import pytest
+
+from tests.gpu_util import step
+
+pytestmark = pytest.mark.gpu
+
+
+# fewer lines than a strip, one and several strips, lines beside the border, one
+# slice (no odd ones), long lines, and lines too long for the strips (colours)
+@pytest.mark.parametrize("M,N,T,bc", [(5, 4, 2, 1), (7, 9, 3, 3), (16, 30, 2, 1), (33, 5, 4, 3), (4, 61, 5, 1),
+                                      (100, 23, 3, 3), (12, 10, 16, 1), (3, 2, 7, 3), (230, 19, 2, 1)])
+def test_strips_match_colours(M, N, T, bc):
+    import torch
+    from spdepy_amd import spdes
+    import spdepy_amd as sp
+    from spdepy_amd.krylov import IterativeSolver
+    ax = lambda n: (np.arange(n) + 0.5) / n
+    g = sp.grid(x=ax(M), y=ax(N), t=np.arange(float(T)))
+    mod0 = spdes.WhittleMatern2D(grid=sp.grid(x=ax(M), y=ax(N)), bc=bc)
+    mod = spdes.AdvectionIDiffusion2D(grid=g, mod0=mod0, bc=bc)
+    eng = mod._engine()
+    q = eng.assemble(mod._coeffs(np.array([0.5, -0.5, 0.4, -0.3, 0.0, 4.0])))
+    it = IterativeSolver(eng.plan)
+    step("strips %dx%dx%d bc %d" % (M, N, T, bc))
+    it.factor(q, torch.full((eng.n,), 50.0, dtype=torch.float64, device="cuda"))
+    b = torch.as_tensor(np.random.default_rng(3).normal(size=(eng.n, 1)).astype(np.float32)).cuda()
+    for its in (1, 4):
+        one, _ = it.solve(b, tol=1e-30, maxit=its)
+        two, _ = it.solve(b.repeat(1, 2).contiguous(), tol=1e-30, maxit=its)
+        a, c = one[:, 0].double(), two[:, 0].double()
+        # FP32 recurrences with other orders of summation: 1e-7 an operation
+        assert float((a - c).norm() / c.norm()) <= 1e-5
