@@ -399,10 +399,12 @@ __global__ __launch_bounds__(256) void gemm64_split_kernel(const GemmProb* __res
     gemm_reg_body<TA, TB, VEC, 2, 2, true>(probs, tiles, bases, split, ws);
 }
 
-// PULL: plus the children's update blocks (beta not used).
-// Block b: C tile of tiles[b * split] = alpha * sum_q partial[b * split + q]
-// (q ascending) + beta C, inside the problem and, for lower problems, on or
-// below the diagonal.
+// Block (b, y): quarter y of the C tile of tiles[b * split] = alpha * sum_q
+// partial[b * split + q] (q ascending) + beta C, inside the problem and, for lower
+// problems, on or below the diagonal.  PULL: plus the children's update blocks
+// (beta not used).  Four entries a thread, the partials of four chunks in
+// flight: bound by the latency of its loads (a block per tile with sixteen entries
+// a thread one after another took 10-38 us, more than the chunks it summed).
 template <bool PULL>
 __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmProb* __restrict__ probs,
                                                            const GemmTile* __restrict__ tiles, Bases bases, int split,
@@ -412,21 +414,45 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmProb* __res
   double* C = bases.p[P.c_base] + P.c_off;
   const int m0 = t.tm * 64, n0 = t.tn * 64;
   const bool diag_tile = P.lower && t.tm == t.tn;
-  const double* w = ws + (int64_t)blockIdx.x * split * 4096;
-  for (int e = threadIdx.x; e < 4096; e += 256) {
-    const int m = m0 + (e & 63), n = n0 + (e >> 6);
-    if (m >= P.M || n >= P.N || (diag_tile && m < n)) continue;
-    double acc = 0.0;
-    for (int q = 0; q < split; ++q) acc += w[(int64_t)q * 4096 + e];
+  const int e0 = blockIdx.y * 1024 + threadIdx.x;
+  const double* w = ws + (int64_t)blockIdx.x * split * 4096 + e0;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0}, old[4];
+  const int m = m0 + (e0 & 63);
+  bool in[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int n = n0 + (e0 >> 6) + 4 * u;
+    in[u] = m < P.M && n < P.N && !(diag_tile && m < n);
+    old[u] = !PULL && in[u] && P.beta != 0.0 ? C[m + (int64_t)n * P.ldc] : 0.0;
+  }
+  int q = 0;
+  for (; q + 4 <= split; q += 4) {
+    double v[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[c][u] = w[(q + c) * 4096 + u * 256];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[u] += v[c][u];
+  }
+  for (; q < split; ++q)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[u] += w[q * 4096 + u * 256];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int n = n0 + (e0 >> 6) + 4 * u;
+    if (!in[u]) continue;
     double* c = C + m + (int64_t)n * P.ldc;
-    const double r = P.alpha * acc;
+    const double r = P.alpha * acc[u];
     if constexpr (PULL) {
       const Pull pq = bases.pulls[P.pull];
       const int i = P.pull_row + m, j = P.pull_row + n;
       *c = assembled(bases.p[kFront], r, pq, child_row(bases.inv, pq, 0, i), child_row(bases.inv, pq, 1, i),
                      child_row(bases.inv, pq, 0, j), child_row(bases.inv, pq, 1, j));
     } else {
-      *c = (P.beta == 0.0) ? r : r + P.beta * (*c);
+      *c = P.beta == 0.0 ? r : r + P.beta * old[u];
     }
   }
 }
@@ -560,10 +586,10 @@ void launch_gemm(const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned ld
     double* ws = b.ws + g.ws_off;
     SPDE_GEMM_FORM(gemm64_split_kernel, grid, block, 0, s, g.d_probs, g.d_tiles, b, g.split, ws);
     if (g.pull)
-      hipLaunchKernelGGL(split_reduce_kernel<true>, dim3(g.ntiles / g.split), block, 0, s, g.d_probs, g.d_tiles, b,
+      hipLaunchKernelGGL(split_reduce_kernel<true>, dim3(g.ntiles / g.split, 4), block, 0, s, g.d_probs, g.d_tiles, b,
                          g.split, ws);
     else
-      hipLaunchKernelGGL(split_reduce_kernel<false>, dim3(g.ntiles / g.split), block, 0, s, g.d_probs, g.d_tiles, b,
+      hipLaunchKernelGGL(split_reduce_kernel<false>, dim3(g.ntiles / g.split, 4), block, 0, s, g.d_probs, g.d_tiles, b,
                          g.split, ws);
     return;
   }
