@@ -475,6 +475,62 @@ __global__ void strip_values_kernel(int64_t n, const int32_t* __restrict__ src, 
   const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (e < n) to[e] = src[e] >= 0 ? from[src[e]] : 0.f;
 }
+// The strips' layout of the in-slice entries of each direction: all slots empty,
+// then a thread per row.  bad: a list that is not laid out as the strips read it
+// (adjacent slices first or last as their parity asks, then or before the slice's
+// own, at most the 5 x 5 pattern's).  Nothing is written past a colour's slots.
+struct StripLayout {
+  int M, N, T;
+  int slots;
+  int at[2][9];
+  const int64_t* ptr[2];
+  const int32_t* col[2];
+  int16_t* delta[2];
+  int32_t* src[2];
+  int* bad;
+};
+__global__ void strip_clear_kernel(StripLayout A, int64_t n) {
+  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (e == 0) *A.bad = 0;
+  if (e >= n) return;
+  for (int dir = 0; dir < 2; ++dir) {
+    A.delta[dir][e] = 0;
+    A.src[dir][e] = -1;
+  }
+}
+__global__ void strip_layout_kernel(StripLayout A, int64_t n) {
+  const int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (v >= n) return;
+  const int64_t Ns = (int64_t)A.M * A.N;
+  const int t = (int)(v / Ns), rem = (int)(v % Ns), i = rem % A.M, j = rem / A.M, k = i % 3 + 3 * (j % 3);
+  const int x = cross_count(i, j, A.M, A.N), before = t > 0 ? x : 0, after = t + 1 < A.T ? x : 0;
+  const int cols = class_size(A.M, k % 3), rows = class_size(A.N, k / 3) * cols, row = j / 3 * cols + i / 3;
+  const int64_t first = t * Ns;
+  bool bad = false;
+  for (int dir = 0; dir < 2; ++dir) {
+    const int64_t p0 = A.ptr[dir][v], p1 = A.ptr[dir][v + 1];
+    // lower lists: both adjacent slices of an odd slice first; upper lists of an
+    // even one: the slice before first, the slice after last
+    const int head = dir == 0 ? (t % 2 ? before + after : 0) : (t % 2 ? 0 : before);
+    const int tail = dir == 1 && t % 2 == 0 ? after : 0;
+    const int own = (int)(p1 - p0) - head - tail, room = strip_slots(k, dir);
+    if (own < 0 || own > room) {
+      bad = true;
+      continue;
+    }
+    int64_t s = t * (int64_t)A.slots + A.at[dir][k] + row;
+    for (int64_t p = p0; p < p1; ++p) {
+      const int64_t c = A.col[dir][p];
+      const bool here = c >= first && c < first + Ns;
+      if (here != (p >= p0 + head && p < p1 - tail)) bad = true;
+      if (p < p0 + head || p >= p1 - tail) continue;
+      A.delta[dir][s] = (int16_t)(c - v);
+      A.src[dir][s] = (int32_t)p;
+      s += rows;
+    }
+  }
+  if (bad) *A.bad = 1;
+}
 __global__ __launch_bounds__(kStripThreads) void strip1_kernel(StripArgs A, const float* __restrict__ in,
                                                                float* __restrict__ out) {
   extern __shared__ float strip_lds[];
@@ -1360,39 +1416,26 @@ void ic_apply_strips(spde_ic* ic, const float* r, float* z, float* tmp, hipStrea
   hipLaunchKernelGGL(strip1_kernel, dim3(nstrip * even), dim3(kStripThreads), lds(A.halo), s, A, tmp, z);
 }
 // Lines per strip: about one block per CU over the slices of a parity, at most
-// what 64 KB of LDS hold with the wider border; 0 where three lines do not fit, on
-// periodic lattices, and where the lists are not laid out as the strips read
-// them (checked for every row).
+// what 64 KB of LDS hold with the wider border; 0 where three lines do not fit and on
+// periodic lattices.
 int strip_lines(const spde_ic* ic) {
   const int M = ic->M, N = ic->N, T = ic->T;
   if (ic->pl->lat.bc == 2 || M < 2 || N < 2 || ic->nlow >= (1 << 30) || T > 65535) return 0;
   const int64_t Ns = (int64_t)M * N;
   if ((int64_t)M * 4 * kStripHalo > 4096 || Ns * kStripSlots > INT32_MAX) return 0;  // does not fit, 16-bit cells
-  for (int64_t v = 0; v < ic->n; ++v) {
-    const int t = (int)(v / Ns), rem = (int)(v % Ns), x = cross_count(rem % M, rem / M, M, N);
-    const int before = t > 0 ? x : 0, after = t + 1 < T ? x : 0;
-    const int64_t l0 = ic->h_lptr[v], l1 = ic->h_lptr[v + 1], u0 = ic->h_uptr[v], u1 = ic->h_uptr[v + 1];
-    const int64_t lf = t % 2 ? before + after : 0, uf = t % 2 ? 0 : before, ub = t % 2 ? 0 : after;
-    if (l1 - l0 < lf || u1 - u0 < uf + ub || l1 - l0 - lf > 24 || u1 - u0 - uf - ub > 24) return 0;
-    const int64_t first = t * Ns;
-    auto here = [&](int64_t c) { return c >= first && c < first + Ns; };
-    for (int64_t p = l0; p < l1; ++p)
-      if (here(ic->h_lcol[p]) != (p >= l0 + lf)) return 0;
-    for (int64_t p = u0; p < u1; ++p)
-      if (here(ic->h_ucol[p]) != (p >= u0 + uf && p < u1 - ub)) return 0;
-  }
   int fit = 0;  // longest strip whose block with the wider border (or the whole slice) fits
   while (fit < N && strip_bytes(M, std::min(N, fit + 1 + 4 * kStripHalo)) <= kStripLds) ++fit;
   const int want = (int)(((int64_t)N * ((T + 1) / 2) + 255) / 256);
   const int ny = std::min(std::max(want, 3), fit);
   return ny >= 3 || ny == N ? ny : 0;
 }
-// The strips' layout of the in-slice entries (checked: every entry has a slot).
+// The strips' layout, from the uploaded lists: written by a thread per row on the GPU,
+// which checks every list on the way (a pass over the rows on the host added 20 ms
+// to the 165 ms of a 100 x 100 x 20 handle).
 int build_strips(spde_ic* ic) {
   ic->strip_ny = strip_lines(ic);
   if (!ic->strip_ny) return SPDE_OK;
   const int M = ic->M, N = ic->N, T = ic->T;
-  const int64_t Ns = (int64_t)M * N;
   int64_t at[2][10];
   for (int dir = 0; dir < 2; ++dir) {
     at[dir][0] = 0;
@@ -1405,34 +1448,25 @@ int build_strips(spde_ic* ic) {
     ic->strip_ny = 0;
     return SPDE_OK;
   }
+  StripLayout A{M, N, T, (int)slots, {}, {ic->d_lptr, ic->d_uptr}, {ic->d_lcol, ic->d_ucol}, {}, {}, nullptr};
   for (int dir = 0; dir < 2; ++dir) {
-    std::vector<int16_t> delta(slots * T, 0);
-    std::vector<int32_t> src(slots * T, -1);
-    const auto& ptr = dir == 0 ? ic->h_lptr : ic->h_uptr;
-    const auto& col = dir == 0 ? ic->h_lcol : ic->h_ucol;
-    for (int64_t v = 0; v < ic->n; ++v) {
-      const int64_t t = v / Ns;
-      const int rem = (int)(v % Ns), i = rem % M, j = rem / M, k = i % 3 + 3 * (j % 3);
-      const int64_t rows = (int64_t)class_size(N, k / 3) * class_size(M, k % 3);
-      const int64_t row = (int64_t)(j / 3) * class_size(M, k % 3) + i / 3;
-      int q = 0;
-      for (int64_t p = ptr[v]; p < ptr[v + 1]; ++p) {
-        if (col[p] < t * Ns || col[p] >= (t + 1) * Ns) continue;
-        if (q >= strip_slots(k, dir)) {  // not the 5 x 5 pattern: colour by colour
-          ic->strip_ny = 0;
-          return SPDE_OK;
-        }
-        // the backward direction's slices end at `slots` (they are walked from the end)
-        const int64_t s = t * slots + (dir == 0 ? 0 : slots - at[1][9]) + at[dir][k] + q * rows + row;
-        delta[s] = (int16_t)(col[p] - v);
-        src[s] = (int32_t)p;
-        ++q;
-      }
-    }
-    int rc = upload_vec(&ic->d_edelta[dir], delta);
-    if (!rc) rc = upload_vec(&ic->d_esrc[dir], src);
-    if (rc) return rc;
-    SPDE_HIP(hipMalloc((void**)&ic->d_evalue[dir], sizeof(float) * std::max<int64_t>(slots * T, 1)));
+    SPDE_HIP(hipMalloc((void**)&ic->d_edelta[dir], sizeof(int16_t) * slots * T));
+    SPDE_HIP(hipMalloc((void**)&ic->d_esrc[dir], sizeof(int32_t) * slots * T));
+    SPDE_HIP(hipMalloc((void**)&ic->d_evalue[dir], sizeof(float) * slots * T));
+    A.delta[dir] = ic->d_edelta[dir];
+    A.src[dir] = ic->d_esrc[dir];
+    // the backward direction's slices end at `slots` (they are walked from the end)
+    for (int k = 0; k < 9; ++k) A.at[dir][k] = (int)(at[dir][k] + (dir == 0 ? 0 : slots - at[1][9]));
+  }
+  A.bad = ic->d_status;
+  hipLaunchKernelGGL(strip_clear_kernel, dim3(blocks_of(slots * T)), dim3(256), 0, 0, A, slots * T);
+  hipLaunchKernelGGL(strip_layout_kernel, dim3(blocks_of(ic->n)), dim3(256), 0, 0, A, ic->n);
+  SPDE_HIP(hipGetLastError());
+  int bad = 0;
+  SPDE_HIP(hipMemcpy(&bad, A.bad, sizeof(int), hipMemcpyDeviceToHost));
+  if (bad) {  // colour by colour
+    ic->strip_ny = 0;
+    return SPDE_OK;
   }
   ic->strip_slots = (int)slots;
   // cells of each strip: forward (decreasing class j mod 3) a line of class 1 or 0
@@ -1819,7 +1853,6 @@ int spde_ic_create(spde_plan* pl, spde_ic** out) {
     spde_ic_destroy(ic);
     return code;
   };
-  if ((rc = build_strips(ic))) return fail(rc);
   if ((rc = upload_vec(&ic->d_crow, crow))) return fail(rc);
   if ((rc = upload_vec(&ic->d_lptr, ic->h_lptr))) return fail(rc);
   if ((rc = upload_vec(&ic->d_uptr, ic->h_uptr))) return fail(rc);
@@ -1845,6 +1878,7 @@ int spde_ic_create(spde_plan* pl, spde_ic** out) {
     return fail(SPDE_ERR_ALLOC);
   }
   if ((rc = alloc_small_work(ic))) return fail(rc);
+  if ((rc = build_strips(ic))) return fail(rc);
   *out = ic;
   return SPDE_OK;
 }
