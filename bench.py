@@ -408,8 +408,10 @@ def main():
     kinds = sorted(set(kind_all.tolist()), key=lambda q: -lms[kind_all == q].sum())
     dom = kinds[0]
 
-    dom_name = "gemm%d_kernel<%s, %s>" % (128 if dom & 4 else 64, "true" if dom & 2 else "false",
-                                        "true" if dom & 1 else "false")
+    # a kind is tile and operand order: NT of large tiles holds syrk_pull_kernel's
+    # launches (the SYRKs that write the update blocks) too
+    dom_name = "gemm%d_kernel<%s, %s, true>" % (128 if dom & 4 else 64, "true" if dom & 2 else "false",
+                                              "true" if dom & 1 else "false")
     family = lfl.sum() / (lms.sum() * 1e-3) / 1e12
     # Timed region: only the dominant kernel's launches carry events (HIP
     # events on each launch's own stream), the rest runs undisturbed.

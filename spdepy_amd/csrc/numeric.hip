@@ -605,12 +605,12 @@ void free_launch(GemmLaunch& g) {
 }
 
 // LDS each 64-tile block of the selected inverse's second-stream products
-// (X = L21 Z, Z^T Z, one level ahead of the chain) reserves: 48 KB holds one
-// such block per CU, so the chain's own products on the first stream keep
-// most of the chip.  128-tile launches run at full width: capping them too
-// gained 0.5% of the evaluation rate but slowed each of their launches by a
-// fifth (exact evaluation at 100x100x20, three alternating runs each: no cap
-// 14.72 evals/s, 64-tiles capped 14.78, all capped 14.86).
+// (X = L21 Z, Z^T Z, one level ahead of the chain) reserves, so that the chain's own
+// products on the first stream keep most of the chip: 48 KB allows three such blocks
+// of the register-fed forms per CU, one or two of the staged A^T B form.  Chosen on
+// staged forms (exact evaluation at 100x100x20, alternating runs: no cap 14.72
+// evals/s, 48 KB 14.78, 32 KB slower) and not measured again since.  128-tile
+// launches run at full width: capping them slowed each by a fifth.
 constexpr unsigned kPreLds = 48 * 1024;
 // GEMM launch, bracketed by HIP events when the plan's timing is enabled.
 void run_gemm(spde_plan* pl, const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned lds = 0) {
