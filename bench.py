@@ -472,7 +472,7 @@ def main():
                    "path": "exact"},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP64_TFLOPS, "traffic": measured_traffic(dom_name),
-                     "kernel": dom_name + " (batched FP64 MFMA tile-list GEMM)",
+                     "kernel": dom_name + " (batched FP64 MFMA tile-list GEMM%s)" % (", with syrk_pull_kernel" if dom == 5 else ""),
                      "launches_per_step": int(sel.sum()) // args.steps,
                      "flop_per_launch": dfl[sel].mean(),
                      "algorithmic_bytes_per_launch": dby[sel].mean(),
