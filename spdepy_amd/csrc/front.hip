@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "internal.hpp"
+#include "wait.hpp"
 
 namespace spde {
 
@@ -245,20 +246,18 @@ __device__ __forceinline__ int peek(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 constexpr int kTileDone = 4;
-// Polls before a wait gives up (seconds; a healthy wait takes microseconds).
 // The tickets make every wait end: a task waits only for tasks with lower
-// tickets (checked when the plan is made), which blocks already run.  Giving
-// up raises the stop flag and sets *status to kStalled, every later wait gives
-// up at once, and the factorisation reports an error.
-constexpr int kSpinLimit = 1 << 22;
-struct Waiter {
+// tickets (checked when the plan is made), which blocks already run.  A wait that
+// passes kSpinLimit polls all the same raises the stop flag and sets *status to
+// kStalled, every later wait gives up at once, and the factorisation reports an
+// error.
+struct Waiter : WaitBudget {
   int* stop;
   int* status;
-  int spins = 0;
-  bool gave_up = false;
+  __device__ __forceinline__ Waiter(int* stop_, int* status_) : stop(stop_), status(status_) {}
   // false: keep waiting
   __device__ __forceinline__ bool over() {
-    if (++spins > kSpinLimit) {
+    if (spent()) {
       if ((threadIdx.x & 63) == 0) {
         __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(status, kStalled, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -271,6 +270,7 @@ struct Waiter {
   }
 };
 __device__ __forceinline__ void wait_tile(const int* flag, Waiter& w) {
+  w.begin();
   while (peek(flag) < kTileDone)
     if (w.gave_up || w.over()) break;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -282,6 +282,7 @@ __device__ __forceinline__ int wait_columns(const int* fl, int R, int k0, int k1
   const int lane = threadIdx.x & 63;
   const int k = k0 + (lane & 31), row = lane < 32 ? ia : ib;
   int n;
+  w.begin();
   for (;;) {
     const bool ok = k < k1 && peek(fl + (int64_t)k * R + row) >= kTileDone;
     const unsigned long long m = __ballot(ok);
