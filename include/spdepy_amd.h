@@ -594,6 +594,11 @@ int spde_debug_gemm(int ta, int tb, int M, int N, int K, double alpha, const dou
 /* The 64 x 4 accumulator lanes of one BF16 16x16x16 matrix instruction with
  * A[i][k] = 16 i + k and B = I (out: 256 floats, device). */
 int spde_debug_bf16_probe(float* out, void* stream);
+/* How a solver handle applies its preconditioner (any may be NULL).  lines: lines
+ * per strip of the one-column application, 0 where it goes colour by colour;
+ * filled: 1 if the strips hold the current factor; probe_lds: LDS bytes that a block
+ * of spde_pcg_solve_coeffs reserves at 64 columns. */
+int spde_debug_ic_strips(const spde_ic* ic, int32_t* lines, int32_t* filled, int32_t* probe_lds);
 
 #ifdef __cplusplus
 }

@@ -149,6 +149,7 @@ _SIGS = {
     "spde_adam": (ctypes.c_int, [ctypes.c_int64, vp, vp, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                                  ctypes.c_float, ctypes.c_int, vp, vp, vp, vp]),
     "spde_debug_bf16_probe": (ctypes.c_int, [vp, vp]),
+    "spde_debug_ic_strips": (ctypes.c_int, [vp, c_i32p, c_i32p, c_i32p]),
 }
 
 _lib = None

@@ -1429,6 +1429,22 @@ int strip_lines(const spde_ic* ic) {
   const int ny = std::min(std::max(want, 3), fit);
   return ny >= 3 || ny == N ? ny : 0;
 }
+// Gives the strips up: one column goes colour by colour from now on.
+int drop_strips(spde_ic* ic) {
+  for (void* p : {(void*)ic->d_edelta[0], (void*)ic->d_edelta[1], (void*)ic->d_evalue[0], (void*)ic->d_evalue[1],
+                  (void*)ic->d_esrc[0], (void*)ic->d_esrc[1], ic->d_slists, (void*)ic->d_scell, (void*)ic->d_srow})
+    if (p) hipFree(p);
+  for (int dir = 0; dir < 2; ++dir) {
+    ic->d_edelta[dir] = nullptr;
+    ic->d_evalue[dir] = nullptr;
+    ic->d_esrc[dir] = nullptr;
+  }
+  ic->d_slists = nullptr;
+  ic->d_scell = nullptr;
+  ic->d_srow = nullptr;
+  ic->strip_ny = ic->strip_slots = 0;
+  return SPDE_OK;
+}
 // The strips' layout, from the uploaded lists: written by a thread per row on the GPU,
 // which checks every list on the way (a pass over the rows on the host added 20 ms
 // to the 165 ms of a 100 x 100 x 20 handle).
@@ -1444,15 +1460,15 @@ int build_strips(spde_ic* ic) {
   }
   // the longer of the two directions' slices, for both
   const int64_t slots = std::max(at[0][9], at[1][9]);
-  if (slots * T > INT32_MAX) {
-    ic->strip_ny = 0;
-    return SPDE_OK;
-  }
+  if (slots * T > INT32_MAX) return drop_strips(ic);
   StripLayout A{M, N, T, (int)slots, {}, {ic->d_lptr, ic->d_uptr}, {ic->d_lcol, ic->d_ucol}, {}, {}, nullptr};
   for (int dir = 0; dir < 2; ++dir) {
-    SPDE_HIP(hipMalloc((void**)&ic->d_edelta[dir], sizeof(int16_t) * slots * T));
-    SPDE_HIP(hipMalloc((void**)&ic->d_esrc[dir], sizeof(int32_t) * slots * T));
-    SPDE_HIP(hipMalloc((void**)&ic->d_evalue[dir], sizeof(float) * slots * T));
+    if (hipMalloc((void**)&ic->d_edelta[dir], sizeof(int16_t) * slots * T) != hipSuccess ||
+        hipMalloc((void**)&ic->d_esrc[dir], sizeof(int32_t) * slots * T) != hipSuccess ||
+        hipMalloc((void**)&ic->d_evalue[dir], sizeof(float) * slots * T) != hipSuccess) {
+      (void)hipGetLastError();  // the handle works without them
+      return drop_strips(ic);
+    }
     A.delta[dir] = ic->d_edelta[dir];
     A.src[dir] = ic->d_esrc[dir];
     // the backward direction's slices end at `slots` (they are walked from the end)
@@ -1464,10 +1480,7 @@ int build_strips(spde_ic* ic) {
   SPDE_HIP(hipGetLastError());
   int bad = 0;
   SPDE_HIP(hipMemcpy(&bad, A.bad, sizeof(int), hipMemcpyDeviceToHost));
-  if (bad) {  // colour by colour
-    ic->strip_ny = 0;
-    return SPDE_OK;
-  }
+  if (bad) return drop_strips(ic);
   ic->strip_slots = (int)slots;
   // cells of each strip: forward (decreasing class j mod 3) a line of class 1 or 0
   // beside a needed line of a higher class, backward a line of a higher class
@@ -1503,10 +1516,7 @@ int build_strips(spde_ic* ic) {
           if ((kind == 0 && dir == 1) || (kind == 2 && dir == 0)) continue;  // not swept
           for (int j = 0; j < N; ++j) {
             if (!use[dir][j] || j % 3 != k / 3) continue;
-            if (j < ylo || j >= yhi) {  // the border is too narrow: colour by colour
-              ic->strip_ny = 0;
-              return SPDE_OK;
-            }
+            if (j < ylo || j >= yhi) return drop_strips(ic);  // the border is too narrow
             for (int i = k % 3; i < M; i += 3) {
               cell.push_back((uint16_t)((j - ylo) * M + i));
               row.push_back((int32_t)(j / 3 * class_size(M, k % 3) + i / 3));
@@ -1583,11 +1593,9 @@ void free_shared(spde_ic* ic) {
   for (void* p : {(void*)ic->d_crow, (void*)ic->d_lptr, (void*)ic->d_uptr, (void*)ic->d_lsrc, (void*)ic->d_ulow,
                   (void*)ic->d_lch, (void*)ic->d_lcol, (void*)ic->d_lkey, (void*)ic->d_ucol, (void*)ic->d_l64,
                   (void*)ic->d_dg64,
-                  (void*)ic->d_adiag, (void*)ic->d_l32, (void*)ic->d_u32, (void*)ic->d_dinv, (void*)ic->d_qc32,
-                  (void*)ic->d_edelta[0], (void*)ic->d_edelta[1], (void*)ic->d_evalue[0], (void*)ic->d_evalue[1],
-                  (void*)ic->d_esrc[0], (void*)ic->d_esrc[1], ic->d_slists, (void*)ic->d_scell,
-                  (void*)ic->d_srow})
+                  (void*)ic->d_adiag, (void*)ic->d_l32, (void*)ic->d_u32, (void*)ic->d_dinv, (void*)ic->d_qc32})
     if (p) hipFree(p);
+  drop_strips(ic);
 }
 // A view takes its parent's pattern and factor at the start of every call.
 inline void sync_view(spde_ic* ic) {
@@ -1930,6 +1938,18 @@ int spde_ic_info(const spde_ic* ic, int64_t* nlow, int32_t* ncolours) {
   }
   if (nlow) *nlow = ic->nlow;
   if (ncolours) *ncolours = kColours;
+  return SPDE_OK;
+}
+
+int spde_debug_ic_strips(const spde_ic* ic, int32_t* lines, int32_t* filled, int32_t* probe_lds) {
+  if (!ic) {
+    set_error("spde_debug_ic_strips: invalid argument");
+    return SPDE_ERR_ARG;
+  }
+  if (ic->parent) ic = ic->parent;
+  if (lines) *lines = ic->strip_ny;
+  if (filled) *filled = ic->strip_ny > 0 && ic->factored;
+  if (probe_lds) *probe_lds = (int32_t)kShareLds;
   return SPDE_OK;
 }
 

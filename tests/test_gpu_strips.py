@@ -1,11 +1,21 @@
 """The one-column preconditioner in strips of lines against the colour-by-colour
 sweeps that two equal columns take: the same few PCG iterations."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from tests.gpu_util import step
 
 pytestmark = pytest.mark.gpu
+
+
+def _strips(it):
+    """(lines per strip, whether the strips hold the current factor, LDS of a probe block)."""
+    from spdepy_amd import _native as nat
+    out = [ctypes.c_int32() for _ in range(3)]
+    nat.check(nat.lib().spde_debug_ic_strips(it._h, *[ctypes.byref(x) for x in out]))
+    return [x.value for x in out]
 
 
 # fewer lines than a strip, one and several strips, lines beside the border, one
@@ -25,6 +35,8 @@ def test_strips_match_colours(M, N, T, bc):
     q = eng.assemble(mod._coeffs(np.array([0.5, -0.5, 0.4, -0.3, 0.0, 4.0])))
     it = IterativeSolver(eng.plan)
     step("strips %dx%dx%d bc %d" % (M, N, T, bc))
+    # the route that one column takes: strips, but for the lines too long for them
+    assert (_strips(it)[0] > 0) == (M != 230)
     it.factor(q, torch.full((eng.n,), 50.0, dtype=torch.float64, device="cuda"))
     b = torch.as_tensor(np.random.default_rng(3).normal(size=(eng.n, 1)).astype(np.float32)).cuda()
     for its in (1, 4):
