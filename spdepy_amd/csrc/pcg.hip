@@ -1341,7 +1341,7 @@ int last_colour(const spde_ic* ic) {
 // colour also take their backward step (x_i = z_i / L_ii: no later colour
 // couples to them), which the backward sweep of ic_apply then skips.
 // lds: bytes of LDS each block of the 64-column sweeps reserves (0: none), which
-// caps how many of their blocks a CU holds (kShareLds).
+// caps how many of their blocks a CU holds (probe_lds).
 int ic_fwd(spde_ic* ic, const float* r, float* z, int logk, hipStream_t s, bool fold = false, unsigned lds = 0) {
   const int last = last_colour(ic);
   for (int c = 0; c < kColours; ++c) {
@@ -1617,9 +1617,18 @@ constexpr int kPoll = 16;     // iterations between the host's looks at the acti
 // reserves in spde_pcg_solve_coeffs, whose probe solves run beside another
 // stream's solve (the conditional mean): 32 KB of the CU's 160 KB holds five
 // instead of eight of their blocks per CU and leaves wave slots to the other
-// stream's short launches (iterative log-likelihood at 100x100x20: 2.95 ->
-// 3.35 evals/s; 24 KB 3.11, 40 KB 3.07, 48 KB 2.83).
+// stream's short launches.  That is for a mean that goes colour by colour without LDS
+// (periodic 99x99x20: 166 ms, 189 without the reservation).  A mean in strips needs
+// 21-34 KB a block itself, which five reservations leave no room for, and where the
+// probes are the longer of the two solves the reservation only slows them: from
+// kShareCells cells on they reserve nothing then (100x100x14 320 -> 279 ms,
+// 100x100x20 275 -> 244, 200x200x24 2268 -> 1707; 16, 24, 28 KB 247, 249, 254 at
+// 100x100x20, 40 KB 296).  Below, the mean is about as long and the two differ by
+// 3% either way (60x60x12 80.5 ms with it, 81.7 without; 60x60x28 128.8 and 125.6;
+// 80x80x16 101.7 and 103.3).
 constexpr unsigned kShareLds = 32 * 1024;
+constexpr int64_t kShareCells = 1 << 17;
+unsigned probe_lds(const spde_ic* ic) { return ic->strip_ny > 0 && ic->n >= kShareCells ? 0 : kShareLds; }
 constexpr int kSegMax = 512;  // residual replacement: at most this many iterations between replacements
 
 // One PCG iteration on the handle's work vectors (R, Z, P, Qv) and X.
@@ -1949,7 +1958,7 @@ int spde_debug_ic_strips(const spde_ic* ic, int32_t* lines, int32_t* filled, int
   if (ic->parent) ic = ic->parent;
   if (lines) *lines = ic->strip_ny;
   if (filled) *filled = ic->strip_ny > 0 && ic->factored;
-  if (probe_lds) *probe_lds = (int32_t)kShareLds;
+  if (probe_lds) *probe_lds = (int32_t)spde::probe_lds(ic);
   return SPDE_OK;
 }
 
@@ -2123,7 +2132,7 @@ int spde_pcg_solve_coeffs(spde_ic* ic, const float* B, float* X, int k, double t
     SPDE_HIP(hipMalloc((void**)&ic->d_hist, sizeof(double) * 2 * 64 * cap));
     ic->hist_cap = cap;
   }
-  int rc = pcg_run(ic, B, X, logk, tol, maxit, iters, s, false, ic->d_hist, cap, kShareLds);
+  int rc = pcg_run(ic, B, X, logk, tol, maxit, iters, s, false, ic->d_hist, cap, probe_lds(ic));
   if (rc) return rc;
   std::vector<double> h((size_t)2 * 64 * cap);
   SPDE_HIP(hipMemcpyAsync(h.data(), ic->d_hist, sizeof(double) * h.size(), hipMemcpyDeviceToHost, s));

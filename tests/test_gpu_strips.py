@@ -45,3 +45,16 @@ def test_strips_match_colours(M, N, T, bc):
         a, c = one[:, 0].double(), two[:, 0].double()
         # FP32 recurrences with other orders of summation: 1e-7 an operation
         assert float((a - c).norm() / c.norm()) <= 1e-5
+
+
+# The reservation of the probes' blocks is for a mean that needs no LDS itself:
+# strips, the line in cells, just under it, and a lattice without strips
+@pytest.mark.parametrize("M,N,T,bc,lds", [(64, 64, 32, 1, 0), (64, 64, 31, 1, 32768), (16, 16, 4, 3, 32768),
+                                          (66, 66, 32, 2, 32768)])
+def test_probes_leave_room_for_the_strips(M, N, T, bc, lds):
+    from spdepy_amd.krylov import IterativeSolver
+    from spdepy_amd.plan import Plan
+    it = IterativeSolver(Plan(M, N, T, bc))
+    step("probe blocks %dx%dx%d bc %d" % (M, N, T, bc))
+    lines, _, reserved = _strips(it)
+    assert (lines > 0) == (bc != 2) and reserved == lds
