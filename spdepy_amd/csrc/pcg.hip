@@ -27,11 +27,17 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "internal.hpp"
 
+// Which factor the strips' values are of: one per parent, shared with its views.
+struct StripFill {
+  std::mutex m;
+  uint64_t version = 0;
+};
 // Pattern, colouring and factor of one precision: built by spde_ic_create,
 // written by spde_ic_factor / spde_ic_correct, read by every solve.  A view
 // (spde_ic_view) takes these fields from its parent at each call.
@@ -58,6 +64,8 @@ struct IcShared {
   uint16_t* d_scell = nullptr;
   int32_t* d_srow = nullptr;
   int32_t* d_esrc[2] = {nullptr, nullptr};    // entry of l32 / u32, -1: none
+  uint64_t version = 0;              // of the FP32 factor: counts its changes
+  StripFill* fill = nullptr;
 };
 // Host copies of the lists (spde_ic_export), kept by the handle that built them.
 struct IcHost {
@@ -1532,17 +1540,28 @@ int build_strips(spde_ic* ic) {
   if (!rc) rc = upload_vec(&ic->d_srow, row);
   return rc;
 }
-// The factor's values in that layout, after its FP32 copies are made.
-void fill_strips(spde_ic* ic, hipStream_t s) {
-  if (!ic->strip_ny) return;
+// The factor's values in that layout, at the first one-column solve after the factor
+// changed (two launches; filled with every factor and correction they were 5% of an
+// IC(0) factorisation at 100x100x20, 2.40 -> 2.52 ms, and 14% of a correction, 0.26
+// -> 0.30 ms, also for callers that have 64 columns only).  Solves of a handle and
+// its views start on different streams and threads: the first one fills and waits
+// for the values while the others wait for it.
+int use_strips(spde_ic* ic, hipStream_t s) {
+  if (!ic->strip_ny) return SPDE_OK;
+  std::lock_guard<std::mutex> lock(ic->fill->m);
+  if (ic->fill->version == ic->version) return SPDE_OK;
   const int64_t n = (int64_t)ic->strip_slots * ic->T;
   for (int dir = 0; dir < 2; ++dir)
     hipLaunchKernelGGL(strip_values_kernel, dim3(blocks_of(n)), dim3(256), 0, s, n, ic->d_esrc[dir],
                        dir == 0 ? ic->d_l32 : ic->d_u32, ic->d_evalue[dir]);
+  SPDE_HIP(hipGetLastError());
+  SPDE_HIP(hipStreamSynchronize(s));
+  ic->fill->version = ic->version;
+  return SPDE_OK;
 }
 // z = M^-1 r = (L L^T)^-1 r: forward from r into z, then backward in place,
 // the last colour's two steps in one launch; one right-hand side in strips when
-// the caller has a vector to spare.
+// the caller has a vector to spare (and has called use_strips).
 int ic_apply(spde_ic* ic, const float* r, float* z, int logk, hipStream_t s, unsigned lds = 0, float* tmp = nullptr) {
   if (logk == 0 && tmp && ic->strip_ny > 0) {
     ic_apply_strips(ic, r, z, tmp, s);
@@ -1596,6 +1615,8 @@ void free_shared(spde_ic* ic) {
                   (void*)ic->d_adiag, (void*)ic->d_l32, (void*)ic->d_u32, (void*)ic->d_dinv, (void*)ic->d_qc32})
     if (p) hipFree(p);
   drop_strips(ic);
+  delete ic->fill;
+  ic->fill = nullptr;
 }
 // A view takes its parent's pattern and factor at the start of every call.
 inline void sync_view(spde_ic* ic) {
@@ -1684,6 +1705,7 @@ int pcg_run(spde_ic* ic, const float* B, float* X, int logk, double tol, int max
   const int k = 1 << logk;
   const int64_t n = ic->n, units = n << logk;
   int rc = ensure_work(ic);
+  if (!rc && logk == 0) rc = use_strips(ic, s);
   if (rc) return rc;
   float* R = ic->d_work;
   float* Z = R + n * 64;
@@ -1895,6 +1917,7 @@ int spde_ic_create(spde_plan* pl, spde_ic** out) {
     return fail(SPDE_ERR_ALLOC);
   }
   if ((rc = alloc_small_work(ic))) return fail(rc);
+  ic->fill = new StripFill();
   if ((rc = build_strips(ic))) return fail(rc);
   *out = ic;
   return SPDE_OK;
@@ -1957,7 +1980,10 @@ int spde_debug_ic_strips(const spde_ic* ic, int32_t* lines, int32_t* filled, int
   }
   if (ic->parent) ic = ic->parent;
   if (lines) *lines = ic->strip_ny;
-  if (filled) *filled = ic->strip_ny > 0 && ic->factored;
+  if (filled) {
+    std::lock_guard<std::mutex> lock(ic->fill->m);
+    *filled = ic->strip_ny > 0 && ic->factored && ic->fill->version == ic->version;
+  }
   if (probe_lds) *probe_lds = (int32_t)spde::probe_lds(ic);
   return SPDE_OK;
 }
@@ -2032,6 +2058,7 @@ int spde_ic_correct(spde_ic* ic, const float* corr, double* logdet_m, void* stre
   }
   hipStream_t s = (hipStream_t)stream;
   const int64_t n = ic->n;
+  ic->version++;
   if (corr) {
     hipLaunchKernelGGL(ic_correct_lower_kernel, dim3(blocks_of(n)), dim3(256), 0, s, n, ic->d_lptr, ic->d_lch,
                        ic->d_adiag, corr, ic->d_l64);
@@ -2041,7 +2068,6 @@ int spde_ic_correct(spde_ic* ic, const float* corr, double* logdet_m, void* stre
   hipLaunchKernelGGL(ic_cast_upper_kernel, dim3(blocks_of(ic->nlow)), dim3(256), 0, s, ic->nlow, ic->d_ulow,
                      ic->d_l64, ic->d_u32);
   hipLaunchKernelGGL(ic_cast_diag_kernel, dim3(blocks_of(n)), dim3(256), 0, s, n, ic->d_dg64, ic->d_dinv);
-  fill_strips(ic, s);
   const unsigned g = grid_for(n);
   hipLaunchKernelGGL(logdet_diag_kernel, dim3(g), dim3(256), 0, s, n, ic->d_dg64, ic->d_part);
   hipLaunchKernelGGL(sum_one_kernel, dim3(1), dim3(kRedThreads), 0, s, (int)g, ic->d_part, ic->d_scal + S_X * 64);
@@ -2215,6 +2241,7 @@ int spde_pcg_replace(spde_ic* ic, const double* b, double* x, double tol, double
   }
   hipStream_t s = (hipStream_t)stream;
   int rc = ensure_work(ic);
+  if (!rc) rc = use_strips(ic, s);
   if (rc) return rc;
   spde_plan* pl = ic->pl;
   const int64_t n = ic->n;
@@ -2319,6 +2346,7 @@ int spde_pcg_replace_block(spde_ic* ic, const double* B, double* X, int k, doubl
   }
   hipStream_t s = (hipStream_t)stream;
   int rc = ensure_work(ic);
+  if (!rc && logk == 0) rc = use_strips(ic, s);
   if (rc) return rc;
   spde_plan* pl = ic->pl;
   const int64_t n = ic->n, units = n << logk;
