@@ -210,6 +210,21 @@ int check_args(spde_plan* pl, spde_plan* sp, const spde_coeffs* c, const int64_t
 
 }  // namespace
 
+// The one-slice work of an evaluation on the side stream.  At the end the caller's
+// stream has it behind itself (joined) or, on an error, the host waits for it; then
+// the one-slice plan, which may outlive the plan that owns the side stream, names
+// the caller's stream as the one of its factorisations.
+struct SideWork {
+  LoglikWs* w;
+  spde_plan* sp;
+  hipStream_t s;
+  bool joined = false;
+  ~SideWork() {
+    if (!joined) (void)hipStreamSynchronize(w->side);
+    sp->slots[0].stream = sp->slots[1].stream = s;
+  }
+};
+
 void loglik_release(spde_plan* pl) {
   LoglikWs* w = static_cast<LoglikWs*>(pl->llws);
   if (!w) return;
@@ -265,6 +280,7 @@ int spde_loglik_enqueue(spde_plan* pl, spde_plan* sp, const spde_coeffs* c, cons
   if ((rc = spde_assemble(pl, c, w->qval, s))) return rc;
   SPDE_HIP(hipEventRecord(w->assembled, s));
   SPDE_HIP(hipStreamWaitEvent(w->side, w->assembled, 0));
+  SideWork side_work{w, sp, s};
   // critical path: Q_c factorised here, its selected inverse on the side
   // stream.  The one-slice log|Q| work needs the assembly only: it goes first on
   // the side stream, which would else wait for the factorisation (after mu_c on
@@ -290,6 +306,7 @@ int spde_loglik_enqueue(spde_plan* pl, spde_plan* sp, const spde_coeffs* c, cons
   hipLaunchKernelGGL(quad_rss_kernel, dim3(g1), dim3(256), 0, s, n * r, w->b, w->qmu, m, r, n, w->cols, w->y, w->part);
   SPDE_HIP(hipEventRecord(w->done, w->side));
   SPDE_HIP(hipStreamWaitEvent(s, w->done, 0));
+  side_work.joined = true;
   SPDE_HIP(hipMemcpyAsync(w->res + R_LDQC, pl->slots[1].ld, sizeof(double), hipMemcpyDeviceToDevice, s));
   // adjoint pass (closed-form log|Q| terms from the one-slice selected
   // inverses), then its three trace sums

@@ -82,3 +82,31 @@ def test_adam_trajectory_matches_oracle(small):
     assert np.allclose(np.array(opt.histF), fs_o, rtol=1e-9, atol=0)
     assert np.allclose(xs, xs_o, rtol=0, atol=1e-8 * scale)
     assert np.allclose(res["x"], xp_o, rtol=0, atol=1e-8 * scale)
+
+
+def test_one_slice_plan_outlives_the_space_time_plan(small):
+    """The factorisations of Q0 and B^T B stay readable (spde_factor_finish)
+    when the plan whose evaluation made them is gone."""
+    import ctypes
+    import torch
+    from spdepy_amd import _native as nat
+    from spdepy_amd.engine import OUT_WIDTH
+    from spdepy_amd.plan import Plan, _ptr, _stream
+    c, m = small
+    M, N, T = m._engine().plan.shape
+    pl, sp = Plan(M, N, T, 1), Plan(M, N, 1, 1)
+    coeffs = m._coeffs(c["par"])
+    cols = np.ascontiguousarray(m._obs_cols(), dtype=np.int64)
+    y = np.ascontiguousarray(np.asarray(m.data, dtype=np.float64).reshape(-1))
+    cells = torch.empty(M * N * OUT_WIDTH, dtype=torch.float64, device="cuda")
+    out = nat.LoglikOut()
+    step("evaluation, then its plan destroyed")
+    nat.check(nat.lib().spde_loglik_grad(pl._h, sp._h, ctypes.byref(coeffs.c), cols.ctypes.data, y.ctypes.data,
+                                         cols.size, 1, float(c["par"][-1]), _ptr(cells), ctypes.byref(out),
+                                         _stream(torch)))
+    q0, gram = sp.assemble_spatial(pl, 0), sp.assemble_spatial(pl, 1)
+    torch.cuda.synchronize()
+    del pl
+    step("log-determinants of the one-slice plan")
+    held = [sp.factor_finish(0), sp.factor_finish(1)]
+    assert held == [sp.factor(0, q0), sp.factor(1, gram)]
