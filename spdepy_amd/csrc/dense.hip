@@ -259,7 +259,8 @@ __device__ __forceinline__ void gemm_reg_body(const GemmProb* __restrict__ probs
   const int lr = lane & 15, lk = lane >> 4;
   const int wm = (wave & 1) * 16 * TM, wn = (wave >> 1) * 16 * TN;
   // wave-uniform bases at the tile's first row and column and at kb; the lane
-  // offsets stay below 2^32 (128 rows or 12 columns of one front)
+  // offsets stay below 2^32 (128 rows or 12 columns of one front, 64 columns of a
+  // solution: checked when the launch is made)
   const int64_t lda = (int64_t)P.lda * 8, ldb = (int64_t)P.ldb * 8;
   const char* pa = (const char*)(bases.p[P.a_base] + P.a_off) + (AKC ? m0 * lda + kb * 8ll : m0 * 8ll + kb * lda);
   const char* pb = (const char*)(bases.p[P.b_base] + P.b_off) + (BKC ? n0 * ldb + kb * 8ll : n0 * 8ll + kb * ldb);

@@ -135,6 +135,18 @@ bool operand_ok(int64_t off, int64_t ld, int64_t rows, int64_t cols, int64_t siz
   return off + (rows - 1) + (cols - 1) * ld < size;
 }
 
+// A lane's offsets inside a tile (register-fed products: tile rows or columns with
+// contiguous k, else up to 12 k columns) must fit 32 bits.
+bool lanes_ok(const GemmLaunch& g, const GemmProb& P) {
+  if (g.gemv || (g.ta && !g.tb && g.tile == 64)) return true;  // 64-bit offsets
+  auto span = [](bool kc, int64_t edge, int64_t rows, int64_t ld) {
+    const int64_t last = std::max<int64_t>(std::min(edge, rows) - 1, 0);
+    return kc ? last * ld * 8 + 96 : last * 8 + 12 * ld * 8;
+  };
+  const int64_t most = (int64_t)UINT32_MAX;
+  return span(g.ta, g.tile_m(), P.M, P.lda) <= most && span(!g.tb, g.tile_n(), P.N, P.ldb) <= most;
+}
+
 // Every problem of a launch must touch only its operands' arenas.
 int validate(const GemmLaunch& g, const ArenaSizes& a, const char* what) {
   for (const GemmProb& P : g.h_probs) {
@@ -142,7 +154,7 @@ int validate(const GemmLaunch& g, const ArenaSizes& a, const char* what) {
     const int64_t br = g.tb ? P.N : P.K, bc = g.tb ? P.K : P.N;
     const bool ok = operand_ok(P.a_off, P.lda, ar, ac, a.sz[P.a_base]) &&
                     operand_ok(P.b_off, P.ldb, br, bc, a.sz[P.b_base]) &&
-                    operand_ok(P.c_off, P.ldc, P.M, P.N, a.sz[P.c_base]);
+                    operand_ok(P.c_off, P.ldc, P.M, P.N, a.sz[P.c_base]) && lanes_ok(g, P);
     if (!ok) {
       set_error(std::string("launch plan out of bounds in ") + what);
       return SPDE_ERR_STATE;
@@ -1100,6 +1112,12 @@ int spde_solve(spde_plan* pl, int slot, int mode, double* B, int nrhs, int64_t l
   if (!pl->slots[slot].factored) {
     set_error("spde_solve: slot not factored");
     return SPDE_ERR_STATE;
+  }
+  const int most = solve_columns(pl->sym.n);
+  if (nrhs > most) {
+    for (int c = 0; c < nrhs; c += most)
+      if ((rc = spde_solve(pl, slot, mode, B + c * ldb, std::min(most, nrhs - c), ldb, stream))) return rc;
+    return SPDE_OK;
   }
   hipStream_t s = (hipStream_t)stream;
   PlanExtra* ex = extra(pl);

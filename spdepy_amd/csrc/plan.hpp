@@ -17,6 +17,15 @@ namespace spde {
 enum : int { kDiagSlots = 25, kPrevBase = 25, kNextBase = 34, kSlots = 43, kPrevWide = 43, kNextWide = 68,
              kSlotsWide = 93 };
 
+// Most columns that one solve may have.  The register-fed products form the
+// offsets of a lane's elements inside a tile in 32 bits, and a tile takes up to 64
+// columns of the n x k solution, 8 n bytes apart (plus 96 bytes of rows): from
+// n = 8.5 million on fewer columns fit.
+inline int solve_columns(int64_t n) {
+  const int64_t fit = (((int64_t)1 << 32) - 1 - 96) / (8 * n) + 1;
+  return fit >= 64 ? INT32_MAX : (int)fit;
+}
+
 struct Lattice {
   int M, N, T, bc;            // bc: 1 zero-flux, 2 periodic, 3 Dirichlet
   int wide = 0;               // 1: neighbouring slices coupled through the 5x5 window

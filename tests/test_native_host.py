@@ -1,14 +1,19 @@
-"""Bounded waits of the front factorisation: each wait has the whole limit."""
+"""Host-compilable rules of the native code: each bounded wait of the front
+factorisation has the whole limit, and no solve takes more columns than the lane
+offsets of its products allow."""
 import os
 import subprocess
+
+import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "spdepy_amd", "csrc")
 
 
-def test_waits_do_not_share_their_limit(tmp_path):
-    exe = str(tmp_path / "wait_budget")
-    subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, os.path.join(ROOT, "tests", "native", "wait_budget.cpp"),
+@pytest.mark.parametrize("name", ["wait_budget", "solve_columns"])
+def test_native_rule(tmp_path, name):
+    exe = str(tmp_path / name)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, os.path.join(ROOT, "tests", "native", name + ".cpp"),
                     "-o", exe], check=True, timeout=120)
     r = subprocess.run([exe], stdout=subprocess.PIPE, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout
