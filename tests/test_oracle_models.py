@@ -328,7 +328,10 @@ def test_golden_30x30x10_is_the_oracle():
     import os
     gold = np.load(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "stationary_30x30x10.npz"))
     c = F.stationary()
-    assert np.array_equal(c["idx"], gold["idx"]) and np.array_equal(c["y"], gold["y"])
+    # y holds sparse solves, whose last bits depend on the host's BLAS kernels: equal to
+    # the rounding that the value below is held to
+    assert np.array_equal(c["idx"], gold["idx"])
+    assert np.abs(c["y"] - gold["y"]).max() <= 1e-12 * np.abs(gold["y"]).max()
     Q, dQ = c["model"].makeQ(c["par"], grad=True)
     S = c["grid"].getS(c["idx"])
     like, jac, _ = Mo.loglike(Q.tocsc(), dQ, S, c["y"], c["par"][-1], trace="exact")
