@@ -12,17 +12,15 @@ namespace spde {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 // ----------------------------------------------------------------- GEMM
-// C(M x N) = alpha op(A) op(B) + beta C, column-major, FP64 MFMA.
-// Block tile BM x BN x 16 (64 or 128), four waves in a 2x2 arrangement, each
-// wave (BM/2) x (BN/2) = (BM/32) x (BN/32) MFMA 16x16 tiles.  LDS is double
-// buffered and the next K-slice is prefetched into registers while the
-// current one feeds the MFMAs.  The MFMA computes the transposed tile
-// (B-fragment as the matrix "A" input) so that the 16 lanes of a row group own
-// 16 consecutive rows of one column of C: stores are 128-byte coalesced in
-// column-major memory.  Accumulator layout of v_mfma_f64_16x16x4f64
-// (measured): lane l, register v holds D[l/16 + 4v][l%16].
+// C(M x N) = alpha op(A) op(B) + beta C, column-major, FP64 MFMA over a list of
+// tiles: register-fed (gemm_reg_body), but for 64x64 tiles of A^T B
+// (gemm_tn_body).  The MFMA computes the transposed tile (B-fragment as the matrix
+// "A" input) so that the 16 lanes of a row group own 16 consecutive rows of one
+// column of C: stores are 128-byte coalesced in column-major memory.  Accumulator
+// layout of v_mfma_f64_16x16x4f64 (measured): lane l, register v holds
+// D[l/16 + 4v][l%16].
 // SPLIT: the block computes the chunk t.pad of `split` chunks of the tile's
-// K range (each a multiple of BK deep) and writes the raw 64x64 partial tile
+// K range (each a multiple of 16 deep) and writes the raw 64x64 partial tile
 // to ws + blockIdx.x * 4096 (column-major, ld 64); split_reduce_kernel then
 // applies alpha, beta and the lower-triangle rule.
 // List entry of block b: the dispatcher hands blocks to the eight XCDs in
@@ -37,22 +35,16 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
   return (g << 6) + ((r & 7) << 3) + (r >> 3);
 }
 
-template <bool TA, bool TB, int BM, int BN, bool SPLIT = false>
-__device__ __forceinline__ void gemm_lds_body(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles,
-                                          const Bases& bases, int split = 1, double* __restrict__ ws = nullptr) {
-  constexpr int BK = 16;
-  // LDS layout follows each operand's memory order so that both the global
-  // loads and the LDS stores are contiguous: an operand stored with m (n)
-  // contiguous goes to a k-major tile (pitch BM+16: the four lane groups of a
-  // fragment read land 32 banks apart), a k-contiguous one to an m-major
-  // (n-major) tile with pitch BK+1.
-  constexpr bool AK = !TA, BKM = TB;  // k-major tiles
-  constexpr int PA = AK ? BM + 16 : BK + 1, PB = BKM ? BN + 16 : BK + 1;
-  constexpr int SA = AK ? BK * PA : BM * PA, SB = BKM ? BK * PB : BN * PB;
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
-  constexpr int LA = BM * BK / 256, LB = BN * BK / 256;
-  __shared__ double As[2][SA];
-  __shared__ double Bs[2][SB];
+// A^T B in 64x64 tiles, both operands with contiguous k, staged in LDS: four waves in
+// a 2x2 arrangement, each 32 x 32.  LDS is double buffered and the next 16-deep
+// K-slice is prefetched into registers while the current one feeds the MFMAs; the
+// tiles are m-major (n-major), as they come from memory, with pitch 17.
+template <bool SPLIT>
+__device__ __forceinline__ void gemm_tn_body(const GemmProb* __restrict__ probs, const GemmTile* __restrict__ tiles,
+                                             const Bases& bases, int split = 1, double* __restrict__ ws = nullptr) {
+  constexpr int BM = 64, BN = 64, BK = 16, PITCH = BK + 1, TM = 2, TN = 2, LOADS = BM * BK / 256, STEP = 256 / BK;
+  __shared__ double As[2][BM * PITCH];
+  __shared__ double Bs[2][BN * PITCH];
   const GemmTile t = tiles[SPLIT ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x)];
   const GemmProb P = probs[t.prob];
   const double* __restrict__ A = bases.p[P.a_base] + P.a_off;
@@ -74,44 +66,37 @@ __device__ __forceinline__ void gemm_lds_body(const GemmProb* __restrict__ probs
     kb = k0;
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * WM, wn = (wave >> 1) * WN;
+  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
   const int lr = lane & 15, lk = lane >> 4;
   const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
-  const int am = TA ? tid / BK : tid % BM, ak = TA ? tid % BK : tid / BM;
-  const int bn = TB ? tid % BN : tid / BK, bk = TB ? tid / BN : tid % BK;
-  constexpr int ASTEP_M = TA ? 256 / BK : 0, ASTEP_K = TA ? 0 : 256 / BM;
-  constexpr int BSTEP_N = TB ? 0 : 256 / BK, BSTEP_K = TB ? 256 / BN : 0;
-  auto aidx = [](int k, int m) { return AK ? k * PA + m : m * PA + k; };
-  auto bidx = [](int k, int n) { return BKM ? k * PB + n : n * PB + k; };
+  const int row = tid / BK, col = tid % BK;  // a thread's rows row + q STEP of both tiles, k = col
+  auto at = [](int k, int m) { return m * PITCH + k; };
   d4 acc[TN][TM];
 #pragma unroll
   for (int x = 0; x < TN; ++x)
 #pragma unroll
     for (int y = 0; y < TM; ++y) acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
-  double ra[LA], rb[LB];
+  double ra[LOADS], rb[LOADS];
   auto load = [&](int k0) {
     k0 += kb;
     const bool full = interior && (k0 + BK <= K);
+    const int gk = k0 + col;
 #pragma unroll
-    for (int q = 0; q < LA; ++q) {
-      const int mm = am + q * ASTEP_M, kk = ak + q * ASTEP_K;
-      const int gm = m0 + mm, gk = k0 + kk;
-      const int64_t off = TA ? gk + (int64_t)gm * P.lda : gm + (int64_t)gk * P.lda;
-      ra[q] = (full || (gm < M && gk < K)) ? A[off] : 0.0;
+    for (int q = 0; q < LOADS; ++q) {
+      const int gm = m0 + row + q * STEP;
+      ra[q] = (full || (gm < M && gk < K)) ? A[gk + (int64_t)gm * P.lda] : 0.0;
     }
 #pragma unroll
-    for (int q = 0; q < LB; ++q) {
-      const int nn = bn + q * BSTEP_N, kk = bk + q * BSTEP_K;
-      const int gn = n0 + nn, gk = k0 + kk;
-      const int64_t off = TB ? gn + (int64_t)gk * P.ldb : gk + (int64_t)gn * P.ldb;
-      rb[q] = (full || (gn < N && gk < K)) ? B[off] : 0.0;
+    for (int q = 0; q < LOADS; ++q) {
+      const int gn = n0 + row + q * STEP;
+      rb[q] = (full || (gn < N && gk < K)) ? B[gk + (int64_t)gn * P.ldb] : 0.0;
     }
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < LA; ++q) As[buf][aidx(ak + q * ASTEP_K, am + q * ASTEP_M)] = ra[q];
+    for (int q = 0; q < LOADS; ++q) As[buf][at(col, row + q * STEP)] = ra[q];
 #pragma unroll
-    for (int q = 0; q < LB; ++q) Bs[buf][bidx(bk + q * BSTEP_K, bn + q * BSTEP_N)] = rb[q];
+    for (int q = 0; q < LOADS; ++q) Bs[buf][at(col, row + q * STEP)] = rb[q];
   };
   const int nk = (K - kb + BK - 1) / BK;
   if (nk > 0) {
@@ -124,17 +109,17 @@ __device__ __forceinline__ void gemm_lds_body(const GemmProb* __restrict__ probs
     if (kt + 1 < nk) load((kt + 1) * BK);
     double fa[2][TM], fb[2][TN];
 #pragma unroll
-    for (int mi = 0; mi < TM; ++mi) fa[0][mi] = As[cur][aidx(lk, wm + mi * 16 + lr)];
+    for (int mi = 0; mi < TM; ++mi) fa[0][mi] = As[cur][at(lk, wm + mi * 16 + lr)];
 #pragma unroll
-    for (int ni = 0; ni < TN; ++ni) fb[0][ni] = Bs[cur][bidx(lk, wn + ni * 16 + lr)];
+    for (int ni = 0; ni < TN; ++ni) fb[0][ni] = Bs[cur][at(lk, wn + ni * 16 + lr)];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int f = s & 1;
       if (s < 3) {
 #pragma unroll
-        for (int mi = 0; mi < TM; ++mi) fa[f ^ 1][mi] = As[cur][aidx(4 * (s + 1) + lk, wm + mi * 16 + lr)];
+        for (int mi = 0; mi < TM; ++mi) fa[f ^ 1][mi] = As[cur][at(4 * (s + 1) + lk, wm + mi * 16 + lr)];
 #pragma unroll
-        for (int ni = 0; ni < TN; ++ni) fb[f ^ 1][ni] = Bs[cur][bidx(4 * (s + 1) + lk, wn + ni * 16 + lr)];
+        for (int ni = 0; ni < TN; ++ni) fb[f ^ 1][ni] = Bs[cur][at(4 * (s + 1) + lk, wn + ni * 16 + lr)];
       }
 #pragma unroll
       for (int ni = 0; ni < TN; ++ni)
@@ -176,8 +161,7 @@ __device__ __forceinline__ void gemm_lds_body(const GemmProb* __restrict__ probs
       }
 }
 
-
-// The same product without LDS.  An FP64 MFMA keeps its SIMD busy for 64
+// The product without LDS.  An FP64 MFMA keeps its SIMD busy for 64
 // cycles and consumes two 512-byte fragments, so the matrix cores are fed
 // from L1/L2 directly and no wave ever waits at a barrier.  Each lane loads
 // its own fragment elements: lane (lr, lk) = (lane % 16, lane / 16) holds, for
@@ -194,7 +178,7 @@ __device__ __forceinline__ void gemm_lds_body(const GemmProb* __restrict__ probs
 // 4096^3 NT 58 -> 65, NN 58 -> 67, TN 51 -> 64; 4096 x 1920 x 4096 NT 53 -> 59,
 // NN 54 -> 60, TN 47 -> 66; 64x64 tiles NT 46 -> 56.  With 64x64 tiles and k
 // contiguous in both operands the 16-line loads bound it (38 against 52
-// TFLOP/s), so that form keeps the LDS kernel above.
+// TFLOP/s), so that form is staged (gemm_tn_body).
 template <bool KC, bool VEC, int T>
 __device__ __forceinline__ void load_half(double (&f)[T][4], const uint32_t (&off)[T], const char* base, int64_t ldb,
                                           int h) {
@@ -377,7 +361,7 @@ template <bool TA, bool TB, bool VEC>
 __global__ __launch_bounds__(256) void gemm64_kernel(const GemmProb* __restrict__ probs,
                                                      const GemmTile* __restrict__ tiles, Bases bases) {
   if constexpr (TA && !TB)
-    gemm_lds_body<TA, TB, 64, 64>(probs, tiles, bases);
+    gemm_tn_body<false>(probs, tiles, bases);
   else
     gemm_reg_body<TA, TB, VEC, 2, 2>(probs, tiles, bases);
 }
@@ -395,7 +379,7 @@ __global__ __launch_bounds__(256) void gemm64_split_kernel(const GemmProb* __res
                                                            const GemmTile* __restrict__ tiles, Bases bases, int split,
                                                            double* __restrict__ ws) {
   if constexpr (TA && !TB)
-    gemm_lds_body<TA, TB, 64, 64, true>(probs, tiles, bases, split, ws);
+    gemm_tn_body<true>(probs, tiles, bases, split, ws);
   else
     gemm_reg_body<TA, TB, VEC, 2, 2, true>(probs, tiles, bases, split, ws);
 }

@@ -485,7 +485,6 @@ int build_factor_plan(spde_plan* pl) {
     pl->trtri.push_back(std::move(gz));
   }
   pl->trtri_heights = (int)(pl->trtri.size() / 2);
-  work = std::max<int64_t>(work, pl->lat.Ns() * 60);
   pl->work_doubles = std::max<int64_t>(work, 1);
   const ArenaSizes as = arena_sizes(pl, 1);
   for (auto& L : pl->levels) {

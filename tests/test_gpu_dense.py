@@ -36,8 +36,8 @@ def test_mfma_f64_lane_layout():
                                    (1100, 1060, 40)])
 def test_gemm_matches_numpy(ta, tb, M, N, K, tile):
     """The last shape has more than 64 tiles and a partial last group of 64
-    (306 tiles of 64, 81 of 128): the XCD-grouped block-to-tile mapping must
-    cover every tile once."""
+    (306 tiles of 64x64, 153 or 162 of 128x64 and 64x128, 81 of 128x128): the
+    XCD-grouped block-to-tile mapping must cover every tile once."""
     import torch
     nat = _lib()
     rng = np.random.default_rng(M * 7 + N * 3 + K)
