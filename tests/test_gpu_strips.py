@@ -32,13 +32,31 @@ def _solver(M, N, T, bc):
     return IterativeSolver(eng.plan), q
 
 
-# fewer lines than a strip, one and several strips, lines beside the border, one
-# slice (no odd ones), long lines, and lines too long for the strips (colours)
+# fewer lines than a strip, one and several strips, lines beside the border, long
+# lines, and lines too long for the strips (colours)
 @pytest.mark.parametrize("M,N,T,bc", [(5, 4, 2, 1), (7, 9, 3, 3), (16, 30, 2, 1), (33, 5, 4, 3), (4, 61, 5, 1),
                                       (100, 23, 3, 3), (12, 10, 16, 1), (3, 2, 7, 3), (230, 19, 2, 1)])
 def test_strips_match_colours(M, N, T, bc):
-    import torch
     it, q = _solver(M, N, T, bc)
+    _one_column_matches_two(it, q, M, N, T, bc)
+
+
+# one slice: no odd ones, the two even sweeps alone
+@pytest.mark.parametrize("M,N,bc", [(5, 4, 1), (16, 30, 3), (100, 23, 1)])
+def test_strips_match_colours_on_one_slice(M, N, bc):
+    import torch
+    from spdepy_amd.krylov import IterativeSolver
+    from spdepy_amd.plan import Plan
+    plan = Plan(M, N, 1, bc)
+    indptr, indices = plan.structure()
+    rows = np.repeat(np.arange(plan.n), np.diff(indptr))
+    # symmetric, diagonally dominant, entries that differ along a row and between rows
+    q = np.where(rows == indices, 30.0, -1.0 / (1.0 + 0.01 * (rows + indices)))
+    _one_column_matches_two(IterativeSolver(plan), torch.as_tensor(q).cuda(), M, N, 1, bc)
+
+
+def _one_column_matches_two(it, q, M, N, T, bc):
+    import torch
     step("strips %dx%dx%d bc %d" % (M, N, T, bc))
     # the route that one column takes: strips, but for the lines too long for them
     assert (_strips(it)[0] > 0) == (M != 230)
