@@ -219,7 +219,7 @@ class Engine:
                 side.wait_event(factored)
                 with torch.cuda.stream(side):
                     self.plan.selinv(1, sqc)
-            mu = self.plan.solve(1, b_dev)
+            mu = self.plan.solve(1, b_dev, overwrite=True)
             qmu = self.plan.spmv(qval, mu)
         else:
             # the reference's route: Q factorised (and inverted) on the side stream
@@ -237,7 +237,7 @@ class Engine:
                 side.wait_event(factored)
                 with torch.cuda.stream(side):
                     self.plan.selinv(1, sqc)
-            mu = self.plan.solve(1, b_dev)
+            mu = self.plan.solve(1, b_dev, overwrite=True)
             qmu = self.plan.spmv(qval, mu)
         resid = obs["y"] - mu[obs["cols"]]
         done = torch.cuda.Event()
@@ -416,7 +416,7 @@ class KronEngine:
             side.wait_event(factored)
             with torch.cuda.stream(side):
                 self.plan.selinv(1, sig_c)
-        mu = self.plan.solve(1, obs["sty"] * tau)
+        mu = self.plan.solve(1, obs["sty"] * tau, overwrite=True)
         qmu = self.plan.spmv(qval, mu)
         resid = obs["y"] - mu[obs["cols"]]
         done = torch.cuda.Event()

@@ -147,11 +147,15 @@ class Plan:
         self.slot_owner[slot] = owner
         return ld.value
 
-    def solve(self, slot, B, mode=nat.SOLVE_A):
-        """B: (n,) or (n, k) float64 cuda tensor; returns a new tensor."""
+    def solve(self, slot, B, mode=nat.SOLVE_A, overwrite=False):
+        """B: (n,) or (n, k) float64 cuda tensor; returns a new tensor.
+        overwrite: the result may take B's memory (one column is solved in
+        place then)."""
         import torch
         one = B.dim() == 1
         X = (B.reshape(-1, 1) if one else B).t().contiguous()  # (k, n) row-major = column-major (n, k)
+        if not overwrite and X.data_ptr() == B.data_ptr():  # no copy was needed for the layout
+            X = X.clone()
         nat.check(nat.lib().spde_solve(self._h, slot, mode, _ptr(X), X.shape[0], self.n, _stream(torch)))
         return X.reshape(-1) if one else X.t()
 

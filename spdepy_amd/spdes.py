@@ -159,7 +159,8 @@ class Factor:
         self._ensure()
         arr = np.asarray(b, dtype=np.float64)
         one = arr.ndim == 1
-        x = self.engine.plan.solve(self.slot, torch.as_tensor(arr.reshape(arr.shape[0], -1)).cuda(), mode)
+        x = self.engine.plan.solve(self.slot, torch.as_tensor(arr.reshape(arr.shape[0], -1)).cuda(), mode,
+                                   overwrite=True)
         out = x.cpu().numpy()
         return out.reshape(-1) if one else out
 

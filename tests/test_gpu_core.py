@@ -178,18 +178,19 @@ def test_closed_form_and_factorised_logdet_agree(case):
     assert np.allclose(j1, j2, rtol=1e-10, atol=1e-10 * np.abs(j2).max())
 
 
-def test_loglike_hutchinson_same_probes():
+@pytest.mark.parametrize("nh1", [20, 1])
+def test_loglike_hutchinson_same_probes(nh1):
     c = CASES["var_b1"]()
     g = c["grid"]
     S = g.getS(c["idx"])
     Qo, dQo = c["model"].makeQ(c["par"], grad=True)
-    V = Mo.reference_probes(g.n, 20, seed=11)
+    V = Mo.reference_probes(g.n, nh1, seed=11)
     like_o, jac_o, _ = Mo.loglike(Qo, dQo, S, c["y"], c["par"][-1], trace="hutchinson", probes=V)
     m = product_case(c)
     m.initFit(c["y"], idx=c["idx"], fitQ0=False)
     np.random.seed(11)
     step("logLike hutchinson")
-    like, jac = m.logLike(c["par"], nh1=20, trace="hutchinson")
+    like, jac = m.logLike(c["par"], nh1=nh1, trace="hutchinson")
     assert abs(like - like_o) <= 1e-9 * abs(like_o)
     scale = np.abs(jac_o).max()
     assert np.allclose(jac, jac_o, rtol=1e-9, atol=1e-9 * scale)

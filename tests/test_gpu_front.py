@@ -57,3 +57,19 @@ def test_front_factorisation_reports_the_pivot(M, N, at):
     step("front %dx%d negative pivot %d" % (M, N, at))
     with pytest.raises(nat.NotPositiveDefinite, match="lattice index %d\\)" % k):
         plan.factor(0, torch.as_tensor(q).cuda())
+
+
+# one column needs no change of layout: the right-hand side must still be the caller's
+@pytest.mark.parametrize("shape", [(), (1,), (2,)])
+def test_solve_leaves_its_right_hand_side(shape):
+    import torch
+    from spdepy_amd.plan import Plan
+    plan = Plan(7, 9, 2, 3)
+    q, A = _spd(plan, 4)
+    plan.factor(0, torch.as_tensor(q).cuda())
+    b = np.random.default_rng(5).normal(size=(plan.n,) + shape)
+    B = torch.as_tensor(b).cuda()
+    step("solve of shape %s" % (b.shape,))
+    X = plan.solve(0, B)
+    assert np.array_equal(B.cpu().numpy(), b)
+    assert np.abs(A @ X.cpu().numpy() - b).max() <= 1e-11 * np.abs(b).max()
