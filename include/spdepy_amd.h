@@ -74,6 +74,11 @@ typedef struct spde_plan spde_plan;
  * spde_assemble_kron only. */
 #define SPDE_PLAN_WIDE_TIME 2
 
+/* front_doubles, z_doubles: a slot's arenas on the device (doubles), where every
+ * front's own columns are padded to a multiple of 64 and its leading dimension to one
+ * of 16, so small leaf_max cost memory (a 300 x 300 slice: 0.8 GB of fronts with
+ * leaf_max 128, 1.2 GB with 16).  The exported symbolic analysis below is of the
+ * compact fronts instead (node q: an n x n block at foff[q]), at most as large. */
 typedef struct spde_plan_info {
   int64_t n, nnz_struct, nnz_L, front_doubles, z_doubles;
   int64_t nnodes, nlevels, max_front, max_p;
@@ -89,8 +94,8 @@ int spde_plan_get_info(const spde_plan* plan, spde_plan_info* info);
 /* Host copies of the structure and the symbolic analysis (for inspection):
  * indptr[n+1], indices[nnz], code[nnz]; perm[n]; nodes[nnodes*8] = (start,
  * p, n, parent, child0, child1, level, nB); foff[nnodes]; bnd[sum nB];
- * relpos[sum nB]; map[nnz] (front-arena offset of each structural entry, -1
- * for the upper triangle).  Any pointer may be NULL. */
+ * relpos[sum nB]; map[nnz] (offset of each structural entry in the compact
+ * fronts, -1 for the upper triangle).  Any pointer may be NULL. */
 int spde_plan_export(const spde_plan* plan, int64_t* indptr, int32_t* indices, uint8_t* code,
                      int32_t* perm, int32_t* nodes, int64_t* foff, int32_t* bnd,
                      int32_t* relpos, int64_t* map);
@@ -204,7 +209,9 @@ int spde_factor_finish(spde_plan* plan, int slot, double* logdet);
  * 3 P B and 4 P^T B (CHOLMOD's apply_P / apply_Pt; these need no factor),
  * 5 L^-1 B and 6 L^-T B (CHOLMOD's solve_L / solve_Lt with
  * use_LDLt_decomposition=False: B and the result in elimination order).
- * B device, n x nrhs column-major with leading dimension ldb, overwritten. */
+ * B device, n x nrhs column-major with leading dimension ldb, overwritten.  From
+ * n = 8.5 million on more than some sixty columns (fewer at larger n) are solved
+ * in several passes over the factor. */
 #define SPDE_SOLVE_A 0
 #define SPDE_SOLVE_L 1
 #define SPDE_SOLVE_LT 2

@@ -618,10 +618,11 @@ void free_launch(GemmLaunch& g) {
 // LDS each 64-tile block of the selected inverse's second-stream products
 // (X = L21 Z, Z^T Z, one level ahead of the chain) reserves, so that the chain's own
 // products on the first stream keep most of the chip: 48 KB allows three such blocks
-// of the register-fed forms per CU, one or two of the staged A^T B form.  Chosen on
-// staged forms (exact evaluation at 100x100x20, alternating runs: no cap 14.72
-// evals/s, 48 KB 14.78, 32 KB slower) and not measured again since.  128-tile
-// launches run at full width: capping them slowed each by a fifth.
+// of the register-fed forms per CU, one or two of the staged A^T B form.  Exact
+// evaluation at 100x100x20 and 60x60x12, two alternating runs each on one card: 48 KB
+// 60.7 and 61.0, 7.0 and 7.2 ms; none 61.2 and 61.5, 7.3 and 7.3; 32 KB 61.4 and
+// 61.0, 7.3 and 7.0; 64 KB 60.8 and 61.4, 7.0 and 7.1.  (Capping the 128-tile launches
+// too slowed each by a fifth on the staged products: they run at full width.)
 constexpr unsigned kPreLds = 48 * 1024;
 // GEMM launch, bracketed by HIP events when the plan's timing is enabled.
 void run_gemm(spde_plan* pl, const GemmLaunch& g, const Bases& b, hipStream_t s, unsigned lds = 0) {

@@ -192,6 +192,19 @@ def test_plan_statistics_100x100x20():
     assert info["max_front"] <= 8000
 
 
+@pytest.mark.parametrize("M,N,T,leaf", [(9, 8, 5, 16), (30, 7, 1, 128), (12, 11, 6, 300)])
+def test_info_gives_the_padded_arenas_and_export_the_compact_fronts(M, N, T, leaf):
+    plan = Plan(M, N, T, 3, leaf_max=leaf, host_only=True)
+    e = plan.export()
+    p, nb = e["nodes"][:, 1].astype(np.int64), e["nodes"][:, 7].astype(np.int64)
+    rows = -(-p // 64) * 64 + nb
+    assert plan.info["front_doubles"] == int((rows * (-(-rows // 16) * 16)).sum())
+    assert plan.info["z_doubles"] == int(((-(-p // 64) * 64) ** 2).sum())
+    compact = int(((p + nb) ** 2).sum())
+    assert e["map"].max() < compact <= plan.info["front_doubles"]
+    assert np.array_equal(e["foff"], np.concatenate([[0], np.cumsum((p + nb) ** 2)[:-1]]))
+
+
 def test_library_exports_every_declared_symbol():
     import re
     import os
