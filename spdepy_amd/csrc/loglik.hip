@@ -213,7 +213,7 @@ int check_args(spde_plan* pl, spde_plan* sp, const spde_coeffs* c, const int64_t
 // The one-slice work of an evaluation on the side stream.  At the end the caller's
 // stream has it behind itself (joined) or, on an error, the host waits for it; then
 // the one-slice plan, which may outlive the plan that owns the side stream, names
-// the caller's stream as the one of its factorisations.
+// the caller's stream as the one of the factorisations made there.
 struct SideWork {
   LoglikWs* w;
   spde_plan* sp;
@@ -221,7 +221,8 @@ struct SideWork {
   bool joined = false;
   ~SideWork() {
     if (!joined) (void)hipStreamSynchronize(w->side);
-    sp->slots[0].stream = sp->slots[1].stream = s;
+    for (Slot& slot : sp->slots)
+      if (slot.stream == w->side) slot.stream = s;
   }
 };
 
