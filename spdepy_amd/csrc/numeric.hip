@@ -68,20 +68,32 @@ void build_layout(spde_plan* pl) {
   pl->lay_z = zoff;
 }
 
-// Scatter map of the device layout from the compact one.
+// Scatter map of the device layout from the compact one (an entry's column is its
+// column variable's place in the node: no division per entry).
 std::vector<int64_t> layout_map(const spde_plan* pl) {
   const Symbolic& sym = pl->sym;
   const Structure& st = pl->st;
-  std::vector<int64_t> map(pl->map.size(), -1);
-  for (size_t r = 0; r + 1 < st.indptr.size(); ++r)
-    for (int64_t e = st.indptr[r]; e < st.indptr[r + 1]; ++e) {
-      if (pl->map[e] < 0) continue;
-      const int q = sym.col_node[sym.iperm[st.indices[e]]];
-      const Node& nd = sym.nodes[q];
-      const FrontLay& f = pl->lay[q];
-      const int64_t at = pl->map[e] - nd.foff, row = at % nd.n(), col = at / nd.n();
-      map[e] = f.foff + (row < nd.p ? row : row - nd.p + f.pp) + col * f.ld;
+  struct Place {
+    int64_t from, to;  // of the node's front in either layout
+    int32_t start, p, n, ld, pad;
+  };
+  std::vector<Place> place(sym.nodes.size());
+  for (size_t q = 0; q < place.size(); ++q) {
+    const Node& nd = sym.nodes[q];
+    const FrontLay& f = pl->lay[q];
+    place[q] = {nd.foff, f.foff, nd.start, nd.p, nd.n(), f.ld, f.pp - nd.p};
+  }
+  std::vector<int64_t> map(pl->map.size());
+  for (size_t e = 0; e < map.size(); ++e) {
+    if (pl->map[e] < 0) {
+      map[e] = -1;
+      continue;
     }
+    const int pc = sym.iperm[st.indices[e]];
+    const Place& f = place[sym.col_node[pc]];
+    const int64_t col = pc - f.start, row = pl->map[e] - f.from - col * f.n;
+    map[e] = f.to + (row < f.p ? row : row + f.pad) + col * f.ld;
+  }
   return map;
 }
 
@@ -778,9 +790,7 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
     return SPDE_OK;
   }
   const Symbolic& sym = pl->sym;
-  const std::vector<int64_t> dmap = layout_map(pl);
-  std::vector<int64_t> dmapsym(dmap.size());
-  for (size_t e = 0; e < dmap.size(); ++e) dmapsym[e] = dmap[e] >= 0 ? dmap[e] : dmap[pl->st.mirror[e]];
+  std::vector<int64_t> dmap = layout_map(pl);
   int rc = SPDE_OK;
 #define TRY(x)                   \
   do {                           \
@@ -802,7 +812,10 @@ int spde_plan_create(int M, int N, int T, int bc, int leaf_max, int nslots, int 
   }
   TRY(upload(&pl->d_diag, pl->st.diag));
   TRY(upload(&pl->d_map, dmap));
-  TRY(upload(&pl->d_mapsym, dmapsym));
+  // in place: the mirror of an upper entry is a lower one, which stays as it is
+  for (size_t e = 0; e < dmap.size(); ++e)
+    if (dmap[e] < 0) dmap[e] = dmap[pl->st.mirror[e]];
+  TRY(upload(&pl->d_mapsym, dmap));
   TRY(upload(&pl->d_perm, sym.perm));
   std::vector<int32_t> relpos(std::max<int64_t>(sym.relpos_total, 1)), bnd(std::max<int64_t>(sym.relpos_total, 1));
   std::vector<NodeDev> nodes(sym.nodes.size());
